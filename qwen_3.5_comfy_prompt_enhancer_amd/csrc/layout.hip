@@ -52,42 +52,67 @@ __global__ void w8_dequant_kernel(const int8_t* __restrict__ w, const void* s, i
 
 // ---------------------------------------------------------------------------
 // Requantization (quant_formats.py:253-275).  Byte and fp32 element work, bound
-// by HBM: every weight is read from HBM once (the second pass of a column's group
-// or of the per-column quantization hits the caches) and its code written once.
+// by HBM: a thread keeps its weights in registers between the amax and the codes, so a
+// weight is read once (columns too long for that are read again from the caches).
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ uint32_t code_w4(float w, float sc) {
-  return (uint32_t)(int)(fminf(fmaxf(rintf(w / sc), -8.0f), 7.0f) + 8.0f);
+// rint(w / sc) with the correctly rounded quotient's value, from a product with
+// inv = fl(1 / sc): the product is within 2^-22 of the quotient relative, 3e-5 for
+// quotients up to 128, so only a product within 1e-4 of a rounding tie needs the division
+// (a division is about twelve instructions; with one per weight these kernels were bound
+// by them, not by HBM).  Infinities and NaN take either form to the same value.
+__device__ __forceinline__ float rint_div(float w, float sc, float inv) {
+  const float t = w * inv;
+  float r = rintf(t);
+  if (__builtin_expect(fabsf(t - r) > 0.4999f, 0)) r = rintf(w / sc);
+  return r;
 }
 
-// W4, 4 columns per thread (N % 4 == 0): 16-byte loads, one 4-byte store per row pair.
-__global__ void requant_w4_x4_kernel(const float* __restrict__ w, int K, int N, int group,
-                                     uint8_t* __restrict__ packed, uint16_t* __restrict__ sbf) {
-  const int n = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+// W4, C columns per thread (N % C == 0), the group's GROUP rows held in registers (C *
+// GROUP = 128 of them): every weight is read once, all of a thread's loads in flight
+// together.  K = 4096, N = 12288, groups of 32 / 64: 42 / 41.5 us (5.4 TB/s), 72 / 79 us
+// with a second read of the rows and a division per weight.
+template <int GROUP, int C>
+__global__ __launch_bounds__(256) void requant_w4_kernel_reg(const float* __restrict__ w, int N,
+                                                             uint8_t* __restrict__ packed,
+                                                             uint16_t* __restrict__ sbf) {
+  typedef float vec __attribute__((ext_vector_type(C)));
+  const int n = C * (blockIdx.x * blockDim.x + threadIdx.x);
   const int gi = blockIdx.y;
   if (n >= N) return;
-  const float* col = w + (long long)gi * group * N + n;
-  f32x4 amax = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int r = 0; r < group; ++r) {
-    const f32x4 v = *(const f32x4*)(col + (long long)r * N);
+  const float* col = w + (long long)gi * GROUP * N;
+  vec v[GROUP];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) amax[c] = fmaxf(amax[c], fabsf(v[c]));
+  for (int r = 0; r < GROUP; ++r)
+    v[r] = __builtin_nontemporal_load((const vec*)(col + (long long)r * N + (uint32_t)n));
+  float sc[C], inv[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    float amax = 0.0f;
+#pragma unroll
+    for (int r = 0; r < GROUP; ++r) amax = fmaxf(amax, fabsf(v[r][c]));
+    sc[c] = fmaxf(amax, 1e-8f) / 7.0f;
+    inv[c] = 1.0f / sc[c];
   }
-  float sc[4];
+  auto code = [&](float x, int c) {
+    return (uint32_t)(int)(fminf(fmaxf(rint_div(x, sc[c], inv[c]), -8.0f), 7.0f) + 8.0f);
+  };
+  uint8_t* prow = packed + (long long)gi * (GROUP / 2) * N;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) sc[c] = fmaxf(amax[c], 1e-8f) / 7.0f;
-  uint8_t* prow = packed + (long long)gi * (group / 2) * N + n;
-  for (int r = 0; r < group; r += 2) {
-    const f32x4 v0 = *(const f32x4*)(col + (long long)r * N);
-    const f32x4 v1 = *(const f32x4*)(col + (long long)(r + 1) * N);
+  for (int r = 0; r < GROUP; r += 2) {
     uint32_t word = 0;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) word |= (code_w4(v0[c], sc[c]) | (code_w4(v1[c], sc[c]) << 4)) << (8 * c);
-    *(uint32_t*)(prow + (long long)(r / 2) * N) = word;
+    for (int c = 0; c < C; ++c) word |= (code(v[r][c], c) | (code(v[r + 1][c], c) << 4)) << (8 * c);
+    uint8_t* d = prow + (long long)(r / 2) * N + (uint32_t)n;
+    if constexpr (C == 4) *(uint32_t*)d = word;
+    else *(uint16_t*)d = (uint16_t)word;
   }
-  *(u32x2*)(sbf + (long long)gi * N + n) =
-      u32x2{(uint32_t)f32_to_bf16(sc[0]) | ((uint32_t)f32_to_bf16(sc[1]) << 16),
-            (uint32_t)f32_to_bf16(sc[2]) | ((uint32_t)f32_to_bf16(sc[3]) << 16)};
+  uint32_t sw[2] = {0u, 0u};
+#pragma unroll
+  for (int c = 0; c < C; ++c) sw[c >> 1] |= (uint32_t)f32_to_bf16(sc[c]) << (16 * (c & 1));
+  uint16_t* sd = sbf + (long long)gi * N + (uint32_t)n;
+  if constexpr (C == 4) *(u32x2*)sd = u32x2{sw[0], sw[1]};
+  else *(uint32_t*)sd = sw[0];
 }
 
 // W4: thread = (group g, column n).  sc = max(amax, 1e-8) / 7 over the group's rows;
@@ -111,7 +136,76 @@ __global__ void requant_w4_kernel(const float* __restrict__ w, int K, int N, int
   sbf[(long long)gi * N + n] = f32_to_bf16(sc);
 }
 
-// W8, pass 1: the bits of max |w| over a block of rows of each column, merged with an
+// W8 in one pass (N % 4 == 0): a workgroup of 1024 threads owns a strip of 4 L columns.
+// Thread (q = tid / L) holds 4 columns of rows q, q + 1024 / L, ... in registers (NIT of
+// them; the rows past those are read again from the caches for the second half), the
+// columns' amax meets in LDS, and the codes are written from the registers.  Bound by HBM,
+// and by a workgroup's read and write phases not overlapping (its registers hold one
+// workgroup per CU).  K = 4096, N = 12288: 76 us, 4096 x 4096: 25 us, 2048 x 2048: 9.0 us,
+// against 110 / 48.5 / 30 us in four launches (amax by atomics, codes with a division
+// each, scale).
+template <int NIT, int L>
+__global__ __launch_bounds__(1024) void requant_w8_strip_kernel(const float* __restrict__ w, int K, int N, int strips,
+                                                                int8_t* __restrict__ q, float* __restrict__ scale) {
+  constexpr int RS = 1024 / L;  // rows per step
+  __shared__ float part[16][4 * L];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // strips narrower than a cache line: neighbours on one XCD (workgroup b runs on XCD b mod 8)
+  const int xcd = (int)blockIdx.x & 7, per8 = strips >> 3, more = strips & 7;
+  const int strip = L < 8 ? xcd * per8 + min(xcd, more) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+  const int c4 = 4 * (tid & (L - 1)), n = 4 * L * strip + c4, r0 = tid / L;
+  const bool valid = n < N;
+  const uint32_t nn = valid ? (uint32_t)n : 0u;
+  f32x4 v[NIT];
+  f32x4 am = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NIT; ++i) {
+    // (a row read twice leaves the amax as it is; a uniform address and a 32-bit offset)
+    const int k0 = RS * i < K ? RS * i : 0;
+    v[i] = *(const f32x4*)(w + (long long)k0 * N + ((uint32_t)min(r0, K - 1 - k0) * (uint32_t)N + nn));
+  }
+#pragma unroll 4
+  for (int r = r0 + RS * NIT; r < K; r += RS) {
+    const f32x4 x = *(const f32x4*)(w + (long long)r * N + nn);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) am[c] = fmaxf(am[c], fabsf(x[c]));
+  }
+#pragma unroll
+  for (int i = 0; i < NIT; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) am[c] = fmaxf(am[c], fabsf(v[i][c]));
+#pragma unroll
+  for (int s = L; s < 64; s <<= 1)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) am[c] = fmaxf(am[c], __shfl_xor(am[c], s));
+  if (lane < L) *(f32x4*)&part[wave][c4] = am;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const f32x4 x = *(const f32x4*)&part[i][c4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) am[c] = fmaxf(am[c], x[c]);
+  }
+  if (!valid) return;
+  f32x4 sc, inv;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) sc[c] = fmaxf(am[c], 1e-8f) / 127.0f, inv[c] = 1.0f / sc[c];
+  if (tid < L) *(f32x4*)(scale + n) = sc;
+  auto put = [&](int k0, const f32x4& x) {  // row k0 + r0
+    uint32_t word = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      word |= ((uint32_t)(int)fminf(fmaxf(rint_div(x[c], sc[c], inv[c]), -127.0f), 127.0f) & 0xFFu) << (8 * c);
+    *(uint32_t*)(q + (long long)k0 * N + ((uint32_t)r0 * (uint32_t)N + nn)) = word;
+  };
+#pragma unroll
+  for (int i = 0; i < NIT; ++i)
+    if (r0 + RS * i < K) put(RS * i, v[i]);
+#pragma unroll 4
+  for (int r = r0 + RS * NIT; r < K; r += RS) put(r - r0, *(const f32x4*)(w + (long long)r * N + nn));
+}
+
+// Any N, pass 1: the bits of max |w| over a block of rows of each column, merged with an
 // unsigned atomic max (the order of non-negative floats is that of their bits) into
 // `bits`, which starts at zero.
 __global__ void w8_amax_kernel(const float* __restrict__ w, int K, int N, int rows, unsigned* __restrict__ bits) {
@@ -121,21 +215,6 @@ __global__ void w8_amax_kernel(const float* __restrict__ w, int K, int N, int ro
   float amax = 0.0f;
   for (int r = r0; r < r1; ++r) amax = fmaxf(amax, fabsf(w[(long long)r * N + n]));
   atomicMax(bits + n, bitcast<unsigned>(amax));
-}
-
-// the same, 4 columns per thread (N % 4 == 0)
-__global__ void w8_amax_x4_kernel(const float* __restrict__ w, int K, int N, int rows, unsigned* __restrict__ bits) {
-  const int n = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
-  if (n >= N) return;
-  const int r0 = blockIdx.y * rows, r1 = min(K, r0 + rows);
-  f32x4 amax = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int r = r0; r < r1; ++r) {
-    const f32x4 v = *(const f32x4*)(w + (long long)r * N + n);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) amax[c] = fmaxf(amax[c], fabsf(v[c]));
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) atomicMax(bits + n + c, bitcast<unsigned>(amax[c]));
 }
 
 __global__ void fill_u32_kernel(unsigned* __restrict__ p, int n, unsigned v) {
@@ -152,26 +231,6 @@ __global__ void w8_quant_kernel(const float* __restrict__ w, int K, int N, const
     const int n = (int)(i % N);
     const float sc = fmaxf(bitcast<float>(bits[n]), 1e-8f) / 127.0f;
     q[i] = (int8_t)(int)fminf(fmaxf(rintf(w[i] / sc), -127.0f), 127.0f);
-  }
-}
-
-__device__ __forceinline__ uint32_t code_w8(float w, float sc) {
-  return (uint32_t)(int)fminf(fmaxf(rintf(w / sc), -127.0f), 127.0f) & 0xFFu;
-}
-
-// the same, 4 consecutive elements per thread (N % 4 == 0, so they share a row)
-__global__ void w8_quant_x4_kernel(const float* __restrict__ w, int K, int N, const unsigned* __restrict__ bits,
-                                   int8_t* __restrict__ q) {
-  const long long total4 = (long long)K * N / 4;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total4;
-       i += (long long)gridDim.x * blockDim.x) {
-    const int n = (int)((4 * i) % N);
-    const f32x4 v = *(const f32x4*)(w + 4 * i);
-    const u32x4 b = *(const u32x4*)(bits + n);
-    uint32_t word = 0;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) word |= code_w8(v[c], fmaxf(bitcast<float>(b[c]), 1e-8f) / 127.0f) << (8 * c);
-    *(uint32_t*)(q + 4 * i) = word;
   }
 }
 
@@ -219,65 +278,85 @@ __global__ void repack_gptq_x4_kernel(const uint32_t* __restrict__ qw, int K, in
   }
 }
 
-// thread = (packed row r, word c): rows 2r and 2r+1 of word column c -> 8 pair bytes
+// rows 2r and 2r+1 of word column c -> 8 pair bytes: byte b of `e` pairs the words'
+// nibbles 2b (columns 0, 4, 1, 5 for b = 0, 1, 2, 3), byte b of `o` their nibbles 2b + 1
+// (columns 2, 6, 3, 7).
+__device__ __forceinline__ u32x2 awq_pairs(uint32_t lo, uint32_t hi) {
+  const uint32_t e = (lo & 0x0F0F0F0Fu) | ((hi & 0x0F0F0F0Fu) << 4);
+  const uint32_t o = ((lo >> 4) & 0x0F0F0F0Fu) | (hi & 0xF0F0F0F0u);
+  return u32x2{perm(o, e, 0x06040200u), perm(o, e, 0x07050301u)};
+}
+
+// thread = (packed row, word); with W2, two words (an even word count, 16-byte stores).
+// K = 4096, N = 12288: 8.7 us, 10.9 with a shift and a mask per nibble and 8-byte stores.
+template <bool W2>
 __global__ void repack_awq_kernel(const uint32_t* __restrict__ qw, int K, int N, uint8_t* __restrict__ packed) {
-  const int W = N / 8;
-  const long long total = (long long)(K / 2) * W;
+  const int W = N / 8, per = W2 ? W / 2 : W;
+  const long long total = (long long)(K / 2) * per;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
        i += (long long)gridDim.x * blockDim.x) {
-    const long long r = i / W, c = i - r * W;
-    const uint32_t lo = qw[(2 * r) * W + c], hi = qw[(2 * r + 1) * W + c];
-    uint32_t b[2] = {0u, 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int sh = 4 * kAwqRev[j];
-      const uint32_t byte = ((lo >> sh) & 0xFu) | (((hi >> sh) & 0xFu) << 4);
-      b[j >> 2] |= byte << (8 * (j & 3));
+    const long long r = i / per, c = i - r * per;
+    if constexpr (W2) {
+      const u32x2 lo = *(const u32x2*)(qw + (2 * r) * W + 2 * c), hi = *(const u32x2*)(qw + (2 * r + 1) * W + 2 * c);
+      const u32x2 a = awq_pairs(lo.x, hi.x), b = awq_pairs(lo.y, hi.y);
+      *(u32x4*)(packed + r * N + 16 * c) = u32x4{a.x, a.y, b.x, b.y};
+    } else {
+      *(u32x2*)(packed + r * N + 8 * c) = awq_pairs(qw[(2 * r) * W + c], qw[(2 * r + 1) * W + c]);
     }
-    *(u32x2*)(packed + r * N + 8 * c) = u32x2{b[0], b[1]};
   }
 }
 
-// z[g][8c + j] = nibble (awq ? kAwqRev[j] : j) of qzeros[g][c], plus `add`
 // compressed-tensors int4 (quant_formats.py:282-354): weight_packed int32 [N][W], 8
 // straight-order K nibbles per word, one output feature per row.  Byte i of word w
 // holds nibbles k = 8w + 2i (low) and 8w + 2i + 1 (high): exactly the engine's pair
 // byte of packed row 4w + i, column n.  So the engine layout [K/2][N] is the byte
-// transpose of the [N][4W] byte view, cut to K/2 rows.  A 64 x 64 byte tile goes
-// through LDS: loaded as dwords along a source row, stored 16 bytes along N.
-__global__ void repack_ct_kernel(const uint32_t* __restrict__ qw, int N, int W, int KB,
-                                 uint8_t* __restrict__ packed) {
-  __shared__ uint8_t t[64][64 + 4];  // [column n - n0][packed row j - j0]
-  const int n0 = blockIdx.x * 64, j0 = blockIdx.y * 64;
+// transpose of the [N][4W] byte view, cut to K/2 rows.  A tile of 128 columns x 128
+// packed rows goes through LDS: a thread loads 16 bytes of each of 4 source rows (V4: W %
+// 4 == 0 and a 16-byte aligned source; word by word otherwise), transposes them 4 x 4 bytes
+// at a time in registers and writes dwords of 4 columns; packed rows then leave as 128
+// contiguous bytes.  K = 4096, N = 12288: 8.8 us, 16.5 through a 64 x 64 tile of single bytes.
+template <bool V4>
+__global__ __launch_bounds__(256) void repack_ct_kernel(const uint32_t* __restrict__ qw, int N, int W, int KB,
+                                                        uint8_t* __restrict__ packed) {
+  constexpr int T = 128, P = T / 4 + 1;  // row pitch in dwords
+  __shared__ uint32_t t[T * P];          // [packed row j - j0][columns 4 nq .. 4 nq + 3]
+  const int n0 = blockIdx.x * T, j0 = blockIdx.y * T;
   const int tid = threadIdx.x;
   {
-    const int r = tid >> 2, c = (tid & 3) * 16;  // source row n0 + r, bytes j0 + c ...
-    const int n = n0 + r;
-    if (n < N) {
+    const int nq = tid >> 3, jc = 16 * (tid & 7);  // source rows n0 + 4 nq .. + 3, bytes j0 + jc .. + 15
+    const int n = n0 + 4 * nq, wj = (j0 + jc) >> 2;
+    u32x4 v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int j = j0 + c + 4 * q;  // first byte of the word
-        if (j < KB) {
-          const uint32_t v = qw[(long long)n * W + (j >> 2)];
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t* src = qw + (long long)min(n + r, N - 1) * W;
+      if constexpr (V4) {
+        v[r] = *(const u32x4*)(src + min(wj, W - 4));  // (words past the row are not stored)
+      } else {
 #pragma unroll
-          for (int b = 0; b < 4; ++b) t[r][c + 4 * q + b] = (uint8_t)(v >> (8 * b));
-        }
+        for (int q = 0; q < 4; ++q) v[r][q] = src[min(wj + q, W - 1)];
       }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t x[4];
+      tr4(v[0][q], v[1][q], v[2][q], v[3][q], x);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) t[(jc + 4 * q + b) * P + nq] = x[b];
     }
   }
   __syncthreads();
-  const int jr = tid >> 2, c = (tid & 3) * 16;  // packed row j0 + jr, columns n0 + c ...
-  const int j = j0 + jr, n = n0 + c;
-  if (j < KB && n < N) {  // N % 16 == 0: the 16 columns are all in range
-    uint32_t w4[4];
+  const int c = 4 * (tid & 7), n = n0 + 4 * c;  // 16 columns
+  if (n >= N) return;                           // N % 16 == 0: the 16 columns are all in range
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      w4[q] = (uint32_t)t[c + 4 * q][jr] | ((uint32_t)t[c + 4 * q + 1][jr] << 8) |
-              ((uint32_t)t[c + 4 * q + 2][jr] << 16) | ((uint32_t)t[c + 4 * q + 3][jr] << 24);
-    *(u32x4*)(packed + (long long)j * N + n) = u32x4{w4[0], w4[1], w4[2], w4[3]};
+  for (int i = 0; i < 4; ++i) {
+    const int jr = 32 * i + (tid >> 3), j = j0 + jr;
+    if (j >= KB) break;
+    const uint32_t* row = t + jr * P + c;
+    *(u32x4*)(packed + (long long)j * N + n) = u32x4{row[0], row[1], row[2], row[3]};
   }
 }
 
+// z[g][8c + j] = nibble (awq ? kAwqRev[j] : j) of qzeros[g][c], plus `add`
 __global__ void zeros_unpack_kernel(const uint32_t* __restrict__ qz, int G, int N, int awq, int add,
                                     uint8_t* __restrict__ z) {
   const long long total = (long long)G * N;
@@ -319,29 +398,41 @@ hipError_t launch_w8_dequant(const int8_t* w, const void* s, int sdt, int K, int
 
 hipError_t launch_requant_w4(const float* w, int K, int N, int group, uint8_t* packed, uint16_t* sbf,
                              hipStream_t st) {
-  if (N % 4 == 0 && aligned16(w) && aligned16(packed) && aligned16(sbf))
-    hipLaunchKernelGGL(requant_w4_x4_kernel, dim3((unsigned)((N / 4 + 255) / 256), (unsigned)(K / group)), dim3(256),
-                       0, st, w, K, N, group, packed, sbf);
+  const dim3 wg(256);
+  if (N % 4 == 0 && group == 32 && aligned16(w) && aligned16(packed) && aligned16(sbf))
+    hipLaunchKernelGGL((requant_w4_kernel_reg<32, 4>), dim3((unsigned)((N / 4 + 255) / 256), (unsigned)(K / 32)), wg,
+                       0, st, w, N, packed, sbf);
+  else if (N % 2 == 0 && group == 64 && aligned16(w) && aligned16(packed) && aligned16(sbf))
+    hipLaunchKernelGGL((requant_w4_kernel_reg<64, 2>), dim3((unsigned)((N / 2 + 255) / 256), (unsigned)(K / 64)), wg,
+                       0, st, w, N, packed, sbf);
   else
-    hipLaunchKernelGGL(requant_w4_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)(K / group)), dim3(256), 0,
-                       st, w, K, N, group, packed, sbf);
+    hipLaunchKernelGGL(requant_w4_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)(K / group)), wg, 0, st, w, K, N,
+                       group, packed, sbf);
   return hipGetLastError();
 }
 
 hipError_t launch_requant_w8(const float* w, int K, int N, int8_t* q, float* scale, hipStream_t st) {
+  if (N % 4 == 0 && aligned16(w) && aligned16(q) && aligned16(scale)) {
+    // 64 columns per strip where that leaves at least 128 strips, or where a strip's rows fit
+    // the registers twice over; 16 columns otherwise (K = 4096: N = 6144 38 us against 46
+    // with 64 columns, N = 8192 65 against 53, N = 16384 150 against 110; K = 1024, N = 6144
+    // 19.4 against 13.0)
+    const bool wide = N >= 8192 || (K <= 1024 && N >= 4096);
+    const int strips = (N + (wide ? 63 : 15)) / (wide ? 64 : 16);
+    const dim3 grid((unsigned)strips), wg(1024);
+    if (wide) hipLaunchKernelGGL((requant_w8_strip_kernel<8, 16>), grid, wg, 0, st, w, K, N, strips, q, scale);
+    else if (K <= 1024) hipLaunchKernelGGL((requant_w8_strip_kernel<4, 4>), grid, wg, 0, st, w, K, N, strips, q, scale);
+    else if (K <= 2048) hipLaunchKernelGGL((requant_w8_strip_kernel<8, 4>), grid, wg, 0, st, w, K, N, strips, q, scale);
+    else hipLaunchKernelGGL((requant_w8_strip_kernel<16, 4>), grid, wg, 0, st, w, K, N, strips, q, scale);
+    return hipGetLastError();
+  }
   unsigned* bits = (unsigned*)scale;  // amax bits first, the scale at the end
   const unsigned cb = (unsigned)((N + 255) / 256);
   constexpr int kRows = 64;  // rows per amax block: enough blocks to fill the chip
   hipLaunchKernelGGL(fill_u32_kernel, dim3(cb), dim3(256), 0, st, bits, N, 0u);
-  if (N % 4 == 0 && aligned16(w) && aligned16(q) && aligned16(scale)) {
-    hipLaunchKernelGGL(w8_amax_x4_kernel, dim3((unsigned)((N / 4 + 255) / 256), (unsigned)((K + kRows - 1) / kRows)),
-                       dim3(256), 0, st, w, K, N, kRows, bits);
-    hipLaunchKernelGGL(w8_quant_x4_kernel, grid_for((long long)K * N / 4), dim3(256), 0, st, w, K, N, bits, q);
-  } else {
-    hipLaunchKernelGGL(w8_amax_kernel, dim3(cb, (unsigned)((K + kRows - 1) / kRows)), dim3(256), 0, st, w, K, N,
-                       kRows, bits);
-    hipLaunchKernelGGL(w8_quant_kernel, grid_for((long long)K * N), dim3(256), 0, st, w, K, N, bits, q);
-  }
+  hipLaunchKernelGGL(w8_amax_kernel, dim3(cb, (unsigned)((K + kRows - 1) / kRows)), dim3(256), 0, st, w, K, N, kRows,
+                     bits);
+  hipLaunchKernelGGL(w8_quant_kernel, grid_for((long long)K * N), dim3(256), 0, st, w, K, N, bits, q);
   hipLaunchKernelGGL(w8_scale_kernel, dim3(cb), dim3(256), 0, st, N, bits);
   return hipGetLastError();
 }
@@ -357,15 +448,21 @@ hipError_t launch_repack_gptq(const int32_t* qw, int K, int N, uint8_t* packed, 
 }
 
 hipError_t launch_repack_awq(const int32_t* qw, int K, int N, uint8_t* packed, hipStream_t st) {
-  hipLaunchKernelGGL(repack_awq_kernel, grid_for((long long)(K / 2) * (N / 8)), dim3(256), 0, st,
-                     (const uint32_t*)qw, K, N, packed);
+  const uint32_t* q = (const uint32_t*)qw;
+  const long long words = (long long)(K / 2) * (N / 8);
+  if (N % 16 == 0 && aligned16(qw) && aligned16(packed))
+    hipLaunchKernelGGL(repack_awq_kernel<true>, grid_for(words / 2), dim3(256), 0, st, q, K, N, packed);
+  else
+    hipLaunchKernelGGL(repack_awq_kernel<false>, grid_for(words), dim3(256), 0, st, q, K, N, packed);
   return hipGetLastError();
 }
 
 hipError_t launch_repack_ct(const int32_t* qw, int N, int W, int K, uint8_t* packed, hipStream_t st) {
   const int KB = K / 2;
-  hipLaunchKernelGGL(repack_ct_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)((KB + 63) / 64)), dim3(256), 0, st,
-                     (const uint32_t*)qw, N, W, KB, packed);
+  const uint32_t* q = (const uint32_t*)qw;
+  const dim3 grid((unsigned)((N + 127) / 128), (unsigned)((KB + 127) / 128)), wg(256);
+  if (W % 4 == 0 && aligned16(qw)) hipLaunchKernelGGL(repack_ct_kernel<true>, grid, wg, 0, st, q, N, W, KB, packed);
+  else hipLaunchKernelGGL(repack_ct_kernel<false>, grid, wg, 0, st, q, N, W, KB, packed);
   return hipGetLastError();
 }
 
