@@ -107,55 +107,117 @@ void plan_override(const Problem& P, int& cols, int& waves, int& upw) {
 // scale, acc) from zero, in increasing K); split value = lane 0 + lane 1; total =
 // ((v0 + v1) + v2) + ...; then the W8 column scale (and residual, one rounding).
 // The 16-row skinny tiles reproduce it with two waves per split (lanes == 2).
-// S is chosen for the engine's 512-row chunk and then held for every M.
+// S is chosen for the engine's 512-row chunk and a 128-row prompt, then held for every M.
 // Calls with fewer rows (decode: one sequence, or up to eight best-of candidates,
 // engine.py:392) run the engine decode work units (echain.hip), whose results depend
 // on (K, N) and the call kind only, so batch rows equal single rows; a chunk remainder
 // of 1-8 rows therefore agrees with the unchunked prefill to the tolerance, not bit
 // for bit.
 constexpr int kRowsM = kDecodeRowsMax + 1;
-constexpr int kRefChunkM = 512;
+constexpr int kRefChunkM = 512, kRefShortM = 128;
 
-// Column tiles of 128 over the call's column ranges.
-long long tiles128(const Problem& P, const SkArgs& a) {
+// Column tiles of `tn` over the call's column ranges.
+long long col_tiles(const Problem& P, const SkArgs& a, int tn) {
   long long t = 0;
-  for (int s = 0; s < (P.epi == EPI_STORE ? a.nseg : 1); ++s) t += (a.seg[s].n + 127) / 128;
+  for (int s = 0; s < (P.epi == EPI_STORE ? a.nseg : 1); ++s) t += (a.seg[s].n + tn - 1) / tn;
   return t;
 }
 
-// Time models of the two kernel families for an engine call of M rows split S ways,
-// fitted to MI355X measurements (both families forced, M = 17-512, W8 and W4-g128, the
-// layer shapes 2048x2048, 6144x2048, 2048x8192 and gate/up 2048x6144, weights rotated
-// over 600 MB so they stream from HBM):
-//   tiled: 7 us + rounds of 256 workgroups x 128-wide K stages x weight sets x t_stage,
-//          t_stage = 1.05 us + 2.5 ns per workgroup in the round (W4: 1.8 us + 1.6 ns),
-//          + the split-K exchange (1.45 us per split, 12 ns per workgroup, 0.1 us per MB
-//          of partial tiles)
-//   rows:  5 us + 0.125 us (W4 0.17) per 16-row tile per million weight elements,
-//          + 1.45 us per split
-// t_tiled is negative where the tiled kernel does not cover the call.
-void engine_times(const Problem& P, const SkArgs& a, int M, int S, double* t_tiled, double* t_rows) {
-  const int nb = P.K / 64;
-  *t_tiled = -1.0;
+// Time models (microseconds) of the kernel families of an engine call of M rows split S
+// ways, fitted to MI355X measurements of every tile and of the 16-row tiles (M = 17-700,
+// S = 1, 2, 4, W8 and W4-g128, layer shapes 1024x1024 to 4096x16384 and 12288x4096, gate/up
+// 2048x6144 and 4096x12288, weights rotated so that they stream from HBM):
+//   tiled: t0 + 128-wide K stages x s[q - 1] for each round of q workgroups per CU (`cap` of
+//          them are resident at once) + the split-K exchange, xs per split and xmb per MB of
+//          partial tiles.  4 % rms from the measurements, 15 % at most.
+//   rows:  t0 + 64-wide block pairs x (c0 + c1 x workgroups per CU) + the exchange.  10 % rms.
+struct TileTime {
+  double t0, s[3], xs, xmb;
+  int cap;
+};
+struct RowsTime {
+  double t0, c0, c1, xs, xw;
+};
+constexpr TileTime kTileTime[2][2][I8_TILES] = {
+    // W8: 128x128, 64x64, 96x64, 128x64, 160x64; one weight set, then gate/up
+    {{{6.2, {1.10, 0, 0}, 0.81, 0.394, 1},
+      {4.7, {0.67, 0.90, 1.17}, 0.51, 0.349, 3},
+      {5.5, {0.81, 1.14, 0}, 0.43, 0.389, 2},
+      {6.0, {1.02, 1.42, 0}, 0.54, 0.347, 2},
+      {6.4, {1.15, 1.64, 0}, 0.60, 0.303, 2}},
+     {{7.6, {2.22, 0, 0}, 3.1, 0.81, 1}, {8.7, {1.02, 1.54, 0}, 0, 0.48, 2}, {9.8, {1.36, 1.89, 0}, 0, 0.466, 2}}},
+    // W4
+    {{{5.5, {1.32, 0, 0}, 0.75, 0.375, 1},
+      {5.3, {0.81, 1.11, 1.34}, 0.40, 0.273, 3},
+      {5.7, {1.06, 1.35, 0}, 0.35, 0.372, 2},
+      {6.0, {1.26, 1.60, 0}, 0.44, 0.339, 2},
+      {6.5, {1.53, 2.02, 0}, 0.49, 0.285, 2}},
+     {{8.2, {2.75, 0, 0}, 0.58, 0.459, 1}, {8.5, {1.33, 1.77, 0}, 0, 0.45, 2}, {9.6, {1.70, 2.21, 0}, 0, 0.427, 2}}}};
+constexpr RowsTime kRowsTime[2][2][2] = {  // [W8, W4][one set, gate/up][S = 1, S > 1]
+    {{{4.0, 0.143, 0.264, 0, 0}, {8.1, 0, 0.739, 0.31, 1.085}},
+     {{6.0, 0.648, 0.369, 0, 0}, {12.1, 0.098, 1.589, 0, 2.04}}},
+    {{{5.5, 0.272, 0.208, 0, 0}, {8.6, 0.509, 0.255, 0, 1.91}},
+     {{7.9, 0.471, 0.368, 0, 0}, {5.8, 0.866, 0.688, 0, 6.62}}}};
+// explicit zeros cost an instruction per output and block (measured 1.2-1.3 x per stage)
+constexpr double kZerosFactor = 1.25;
+
+double tile_time(const Problem& P, const SkArgs& a, int tile, int M, int S) {
+  const TileTime& m = kTileTime[P.wk == WK_W4][P.nsets - 1][tile];
+  int bm, bn;
+  prefill_i8_geometry(tile, &bm, &bn);
+  const long long wgs = (long long)((M + bm - 1) / bm) * col_tiles(P, a, bn) * S;
+  const int nst = (P.K / 64 / S + 1) / 2;
+  const long long full = wgs / (256LL * m.cap), rest = wgs - full * 256LL * m.cap;
+  double st = (double)full * m.s[m.cap - 1];
+  if (rest > 0) st += m.s[(rest + 255) / 256 - 1];
+  double t = m.t0 + st * nst * (P.hz ? kZerosFactor : 1.0);
+  if (S > 1) t += m.xs * S + m.xmb * 1e-6 * (double)wgs * bm * bn * 4 * P.nsets;
+  return t;
+}
+
+double rows_time(const Problem& P, const SkArgs& a, int M, int S) {
+  const RowsTime& m = kRowsTime[P.wk == WK_W4][P.nsets - 1][S > 1];
+  const double w = (double)((M + 15) / 16) * col_tiles(P, a, S > 1 ? 128 : 64) * S / 256.0;
+  return m.t0 + (P.K / 64 / S / 2) * (m.c0 + m.c1 * std::max(1.0, w)) * (P.hz ? 1.15 : 1.0) + m.xs * S + m.xw * w;
+}
+
+// Rows per launch that `cap` bytes of partial tiles and the arrival counters hold, in
+// whole tiles of bm rows (every row with one split).
+long long rows_that_fit(const Problem& P, const SkArgs& a, int M, int S, int bm, int bn, size_t cap) {
+  if (S <= 1) return M;
+  const long long nt = col_tiles(P, a, bn);
+  const double row_bytes = (double)S * P.nsets * nt * bn * sizeof(float);
+  const long long cap_rows = (long long)((double)cap / row_bytes) / bm * bm;
+  const long long cnt_rows = (long long)(kCounterBytes / sizeof(unsigned)) / nt * bm;
+  return std::min<long long>(M, std::min(cap_rows, cnt_rows));
+}
+
+// The tile the model prefers for M rows and S splits among those that cover the call and
+// whose partials fit `cap` bytes, -1 if there is none; *t its time.
+int best_tile(const Problem& P, const SkArgs& a, int M, int S, size_t cap, double* t, const char* force = nullptr) {
   SkArgs probe = a;
   probe.M = M;
-  if (prefill_i8_ok(probe, P.wk, P.epi)) {
-    const long long tiles = (long long)((M + 127) / 128) * tiles128(P, a);
-    const long long wgs = tiles * S;
-    const double occ = (double)std::min<long long>(wgs, 256);
-    const double t_stage = (P.wk == WK_W4 ? 1.8e-6 + 1.6e-9 * occ : 1.05e-6 + 2.5e-9 * occ) * P.nsets;
-    double t = 7e-6 + (double)((wgs + 255) / 256) * ((nb / S + 1) / 2) * t_stage;
-    if (S > 1) t += 1.45e-6 * S + 12e-9 * wgs + 0.1e-12 * (double)wgs * P.nsets * 128 * 128 * sizeof(float);
-    *t_tiled = t;
+  int best = -1;
+  const int n = P.epi == EPI_STORE ? I8_TILES : I8_128x64;  // gate/up: the first three
+  for (int k = 0; k < n; ++k) {
+    int bm, bn;
+    prefill_i8_geometry(k, &bm, &bn);
+    if (!prefill_i8_ok(probe, P.wk, P.epi, k) || rows_that_fit(P, a, M, S, bm, bn, cap) < std::min(M, bm)) continue;
+    const double tk = tile_time(P, a, k, M, S);
+    const bool forced = force && *force && atoi(force) == k;
+    if (best < 0 || tk < *t || forced) best = k, *t = tk;
+    if (forced) break;
   }
-  const double elems = (double)P.K * P.ncols * P.nsets / 1e6;
-  *t_rows = 5e-6 + (P.wk == WK_W4 ? 0.17e-6 : 0.125e-6) * ((M + 15) / 16) * elems + (S > 1 ? 1.45e-6 * S : 0.0);
+  return best;
 }
 
 // Split count of the K order: the S (1, 2, 4 or 8, dividing K into ranges of at least
-// two 64-wide blocks) whose faster family is fastest at the engine's 512-row chunk.
-// QLIN_ENGINE_SPLITS overrides it (tuning; it changes the K order).
-int engine_splits(const Problem& P, const SkArgs& a) {
+// two 64-wide blocks) with the least product of the best family's times at the engine's
+// 512-row chunk and at a short prompt of 128 rows.  QLIN_ENGINE_SPLITS overrides it
+// (tuning; it changes the K order).
+int engine_splits(const Problem& call, const SkArgs& a) {
+  Problem P = call;
+  P.hz = false;  // zeros of 8 give the bits of no zeros: the same order for both
   const int nb = P.K / 64;
   const char* es = getenv("QLIN_ENGINE_SPLITS");
   if (es && *es) return atoi(es);
@@ -165,9 +227,12 @@ int engine_splits(const Problem& P, const SkArgs& a) {
   b.x = nullptr;  // the choice must not depend on where the activations sit
   for (int s = 1; s <= 8; s *= 2) {
     if (nb % s != 0 || (s > 1 && nb / s < 2)) break;
-    double tt, tr;
-    engine_times(P, b, kRefChunkM, s, &tt, &tr);
-    const double t = (tt >= 0.0 && tt < tr) ? tt : tr;
+    double t = 1.0;
+    for (const int m : {kRefChunkM, kRefShortM}) {
+      double tt = 0.0;
+      const double tr = rows_time(P, b, m, s);
+      t *= best_tile(P, b, m, s, kWorkspaceBytes, &tt) >= 0 && tt < tr ? tt : tr;
+    }
     if (s == 1 || t < best) best = t, S = s;
   }
   return S;
@@ -252,32 +317,26 @@ int engine_rows(const char* fn, const Problem& P, SkArgs& a, void* workspace, si
   const char* e = getenv("QLIN_ENGINE_PREFILL");
   const bool force_rows = e && strcmp(e, "skinny") == 0;
   const bool force_tiled = e && strcmp(e, "tiled") == 0;
-  // time models of the two families (engine_times) at this M
-  bool tiled = false;
+  const size_t part_cap = (workspace && ws_bytes > kPartBase) ? ws_bytes - kPartBase : 0;
+  int tile = -1;
   if (!force_rows) {
-    double t_tiled, t_rows;
-    engine_times(P, a, P.M, S, &t_tiled, &t_rows);
-    tiled = t_tiled >= 0.0 && (force_tiled || t_tiled < t_rows);
+    double t_tile = 0.0;
+    // (QLIN_I8_TILE forces one tile where it covers the call: the same bits)
+    tile = best_tile(P, a, P.M, S, part_cap, &t_tile, getenv("QLIN_I8_TILE"));
+    if (!force_tiled && tile >= 0 && t_tile >= rows_time(P, a, P.M, S)) tile = -1;
   }
+  const bool tiled = tile >= 0;
   // the tiled kernel has no producer prologue: make the activations first
   if (tiled && a.pro.kind != PRO_NONE) QL_TRY(pro_materialize(fn, a, stream));
-  const int TN = tiled ? 128 : (S == 1 ? 64 : 128);
-  long long ntiles = 0;
-  for (int s = 0; s < (P.epi == EPI_STORE ? a.nseg : 1); ++s) ntiles += (a.seg[s].n + TN - 1) / TN;
+  int rstep = 16, TN = S == 1 ? 64 : 128;
+  if (tiled) prefill_i8_geometry(tile, &rstep, &TN);
+  const long long ntiles = col_tiles(P, a, TN);
   // rows per launch: the split-K partials and arrival counters of a launch must fit
   // the workspace (rows are independent, so blocks of rows give the same bits)
-  const size_t part_cap = (workspace && ws_bytes > kPartBase) ? ws_bytes - kPartBase : 0;
-  const int rstep = tiled ? 128 : 16;
-  long long mb_rows = P.M;
-  if (S > 1) {
-    const double row_bytes = (double)S * P.nsets * ntiles * TN * sizeof(float);  // per row of partials
-    const long long cap_rows = (long long)((double)part_cap / row_bytes) / rstep * rstep;
-    const long long cnt_rows = (long long)(kCounterBytes / sizeof(unsigned)) / ntiles * rstep;
-    mb_rows = std::min<long long>(P.M, std::min(cap_rows, cnt_rows));
-    if (mb_rows < std::min(P.M, rstep))
-      return fail(QLIN_ERR_WORKSPACE, "%s: the workspace (%zu bytes) cannot hold %d K splits of %lld columns", fn,
-                  ws_bytes, S, (long long)ntiles * TN);
-  }
+  const long long mb_rows = rows_that_fit(P, a, P.M, S, rstep, TN, part_cap);
+  if (mb_rows < std::min(P.M, rstep))
+    return fail(QLIN_ERR_WORKSPACE, "%s: the workspace (%zu bytes) cannot hold %d K splits of %lld columns", fn,
+                ws_bytes, S, (long long)ntiles * TN);
   if (clear && S > 1) {
     // one counter per (16-row tile, column tile) at most, for the rows of one launch
     const long long n = ((mb_rows + 15) / 16) * ntiles;
@@ -292,7 +351,7 @@ int engine_rows(const char* fn, const Problem& P, SkArgs& a, void* workspace, si
     hipError_t err;
     if (tiled) {
       if (!b.x || !b.xs) return fail(QLIN_ERR_INVALID, "%s: internal error: no activations for the tiled kernel", fn);
-      err = launch_prefill_i8(b, P.wk, P.hz, P.epi, stream);
+      err = launch_prefill_i8(b, P.wk, P.hz, P.epi, tile, stream);
     } else {
       SkLaunch L;
       L.act = P.act;

@@ -1,0 +1,8 @@
+// The tiled int8-activation kernels for W4 weights with zeros (the kernel is in prefill_i8_kernel.h).
+#include "prefill_i8_kernel.h"
+
+namespace qlin {
+
+template hipError_t launch_i8_w<WK_W4, true>(const SkArgs&, int, int, int, hipStream_t);
+
+}  // namespace qlin

@@ -95,10 +95,13 @@ hipError_t launch_skinny_f16(const SkLaunch& L, const SkArgs& a, hipStream_t str
 hipError_t launch_skinny_i8w8(const SkLaunch& L, const SkArgs& a, hipStream_t stream);
 hipError_t launch_skinny_i8w4(const SkLaunch& L, const SkArgs& a, hipStream_t stream);
 // Tiled int8-activation kernel for the engine-signature calls with more than 16 rows
-// (prefill_i8.hip), store and gate/up epilogues: whether it covers the call (K % 64
-// == 0, W4 groups of at least 64, every column range a multiple of 128), and its launch.
-bool prefill_i8_ok(const SkArgs& a, int wk, int epi);
-hipError_t launch_prefill_i8(SkArgs a, int wk, bool hz, int epi, hipStream_t stream);
+// (prefill_i8.hip), store and gate/up epilogues: its tile shapes (gate/up: the first three),
+// whether it covers the call with one (K % 64 == 0, W4 groups of at least 64, every column
+// range a multiple of the tile's columns), and its launch.
+enum I8Tile { I8_128x128 = 0, I8_64x64, I8_96x64, I8_128x64, I8_160x64, I8_TILES };
+void prefill_i8_geometry(int tile, int* bm, int* bn);
+bool prefill_i8_ok(const SkArgs& a, int wk, int epi, int tile);
+hipError_t launch_prefill_i8(SkArgs a, int wk, bool hz, int epi, int tile, hipStream_t stream);
 
 // Engine-signature call outside the fast kernels' layout rules (edge.hip): any N,
 // pointers aligned to their element size only.  Segments, epilogue and element types
