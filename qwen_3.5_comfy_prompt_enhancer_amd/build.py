@@ -44,6 +44,7 @@ CFLAGS = [
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 EXTRA = {
     "prefill.hip": _VGPR_FORM,
+    "prefill_kg.hip": _VGPR_FORM,
     "prefill_w4_f16.hip": _VGPR_FORM,
     "prefill_w4_bf16.hip": _VGPR_FORM,
     "prefill_w4_f32.hip": _VGPR_FORM,

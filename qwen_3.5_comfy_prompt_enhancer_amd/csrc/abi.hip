@@ -889,9 +889,48 @@ struct PfPlan {
   int shape;
   int splits;
   int sk;  // balanced schedule: K tiles per workgroup (0 = off)
+  int kg;  // rows of the short-prompt kernel's tile (32 or 64), with `splits`; 0: not that kernel
 };
 
-PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap) {
+// Short-prompt kernel (prefill_kg.hip), microseconds: t0 + 32-wide steps of a wave x s[q - 1]
+// for each round of q workgroups per CU (`cap` resident at once) + the bytes its tiles read,
+// mb per MB + the exchange, x0 + xs per split and xmb per MB of partial tiles.  Fitted to
+// MI355X measurements of both tiles with 1, 2, 3, 4, 6 and 8 splits (M = 17-512, shapes
+// 1024x1024 to 4096x12288, weights from HBM): 4-7 % rms, choices within 0.3 % of the best.
+struct KgTime {
+  double t0, s[3], mb, x0, xs, xmb;
+  int cap;
+};
+constexpr KgTime kKgTime[2][2] = {  // [W8, W4][32, 64 rows]
+    {{3.8, {0.27, 0.46, 0.73}, 0.0206, 0.36, 0.41, 0.42, 3}, {4.5, {0.30, 0.62, 0}, 0.0243, 0.28, 0.43, 0.37, 2}},
+    {{4.0, {0.37, 0.44, 0.65}, 0.0149, 0.11, 0.40, 0.41, 3}, {4.8, {0.46, 0.68, 0}, 0.0133, 0.13, 0.42, 0.41, 2}}};
+constexpr long long kKgWorkgroups = 1024;
+
+// The best short-prompt plan of a call: its time in seconds (negative if there is none).
+double plan_kg(int wk, int M, int K, int N, size_t part_cap, PfPlan* plan) {
+  double best = -1.0;
+  for (int k = 0; k < 2; ++k) {
+    const KgTime& m = kKgTime[wk == WK_W4][k];
+    const int bm = 32 << k;
+    const long long tiles = (long long)((M + bm - 1) / bm) * ((N + 63) / 64);
+    const double mb = (double)tiles * K * (2.0 * bm + 64.0 * (wk == WK_W4 ? 0.5 : 1.0)) * 1e-6;
+    for (const int S : {1, 2, 3, 4, 6, 8}) {
+      const long long wgs = tiles * S;
+      const double part = (double)wgs * bm * 64 * sizeof(float);
+      if (wgs > kKgWorkgroups) break;
+      if (S > 1 && (part > (double)part_cap || tiles > (long long)(kCounterBytes / sizeof(unsigned)))) break;
+      const int steps = (K / 32 + 4 * S - 1) / (4 * S);
+      const long long full = wgs / (256LL * m.cap), rest = wgs - full * 256LL * m.cap;
+      double st = (double)full * m.s[m.cap - 1];
+      if (rest > 0) st += m.s[(rest + 255) / 256 - 1];
+      const double t = m.t0 + steps * st + m.mb * mb + (S > 1 ? m.x0 + m.xs * S + m.xmb * part * 1e-6 : 0.0);
+      if (best < 0.0 || t * 1e-6 < best) best = t * 1e-6, *plan = PfPlan{true, 0, S, 0, bm};
+    }
+  }
+  return best;
+}
+
+PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap, bool allow_kg) {
   // Time model fitted to MI355X measurements with the weights streaming from HBM
   // (M = 128 / 512 / 2048 on the 2048x6144, 6144x2048 and 2048x2048 shapes):
   //   tiled:  5 us + rounds x (K tiles per split) x t_tile  (x 1.3 for W4)
@@ -912,7 +951,7 @@ PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap) {
   const double w4f = w4 ? 1.3 : 1.0;
   const Cand cands[2] = {{PF_128x128_K2, 2, {0.48e-6, 1.35e-6}}, {PF_256x256, 1, {1.96e-6, 1.96e-6}}};
   const int nk = K / 64;
-  PfPlan best{false, PF_128x128_K2, 1, 0};
+  PfPlan best{false, PF_128x128_K2, 1, 0, 0};
   const double row_wgs = (double)((M + 15) / 16) * ((N + 127) / 128);
   double best_t = (w4 ? 5.8e-6 : 7.1e-6) + (row_wgs > 256 ? row_wgs / 256 : 1.0) * (w4 ? 2.7e-9 : 3.4e-9) * K;
   for (const Cand& c : cands) {
@@ -932,7 +971,7 @@ PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap) {
                        (S > 1 ? 1.45e-6 * S + 12e-9 * wgs + 0.1e-12 * tile_bytes : 0.0);
       if (t < best_t) {
         best_t = t;
-        best = PfPlan{true, c.shape, S, 0};
+        best = PfPlan{true, c.shape, S, 0, 0};
       }
     }
     // Balanced schedule: every CU slot gets the same run of (tile, K tile) units,
@@ -954,11 +993,16 @@ PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap) {
         const double t = 5e-6 + sk * c.t_tile[occ - 1] * w4f + 2e-6 + 0.22e-12 * xbytes;
         if (t < best_t) {
           best_t = t;
-          best = PfPlan{true, c.shape, 1, sk};
+          best = PfPlan{true, c.shape, 1, sk, 0};
         }
       }
     }
   }
+  // the short-prompt kernel, where its model is 10 % ahead (the models above are off by
+  // about that much): 2048x2048 at M = 128 13.6 -> 8.1 us (W8), 6144x2048 21.5 -> 13.3 (W4)
+  PfPlan kg;
+  const double t_kg = allow_kg ? plan_kg(wk, M, K, N, part_cap, &kg) : -1.0;
+  if (t_kg >= 0.0 && t_kg < 0.9 * best_t) return kg;
   return best;
 }
 
@@ -1038,15 +1082,16 @@ int a16_linear(const char* fn, int wk, const void* x, int x_dtype, int M, int K,
     t.sk = 0;
     t.gm = 0;
     if (fits32) {
-      PfPlan p = plan_prefill(wk, M, K, N, part_cap);
+      PfPlan p = plan_prefill(wk, M, K, N, part_cap, !force_tiled);
       if (getenv("QLIN_PREFILL_VERBOSE"))
         fprintf(stderr, "qlin prefill plan M=%d K=%d N=%d: %s shape=%d splits=%d sk=%d\n", M, K, N,
-                p.tiled ? "tiled" : "skinny", p.shape, p.splits, p.sk);
+                p.kg ? "short" : p.tiled ? "tiled" : "skinny", p.kg ? p.kg : p.shape, p.splits, p.sk);
       const char* e = getenv("QLIN_PREFILL_SHAPE");
       const char* e2 = getenv("QLIN_PREFILL_SPLITS");
       const char* e3 = getenv("QLIN_PREFILL_SK");
       if ((e && *e) || (e2 && *e2) || (e3 && *e3)) {
         p.tiled = true;
+        p.kg = 0;
         if (e && *e) p.shape = atoi(e);
         p.splits = (e2 && *e2) ? atoi(e2) : 1;
         p.sk = (e3 && *e3) ? atoi(e3) : 0;
@@ -1063,6 +1108,24 @@ int a16_linear(const char* fn, int wk, const void* x, int x_dtype, int M, int K,
                           tiles * 2 * waves * 128 * 64 * sizeof(float) > part_cap ||
                           tiles > kCounterBytes / sizeof(unsigned)))
           return fail(QLIN_ERR_UNSUPPORTED, "%s: QLIN_PREFILL_SK=%d unusable here", fn, p.sk);
+      }
+      // QLIN_PREFILL_KG="rows,splits" forces the short-prompt kernel (tuning)
+      const char* ek = getenv("QLIN_PREFILL_KG");
+      int kbm = 0, ksp = 0;
+      if (ek && sscanf(ek, "%d,%d", &kbm, &ksp) == 2) {
+        const size_t tiles = kbm > 0 ? (size_t)((M + kbm - 1) / kbm) * ((N + 63) / 64) : 0;
+        if ((kbm != 32 && kbm != 64) || ksp < 1 || ksp > 64 || tiles * ksp > (1u << 24) ||
+            (ksp > 1 && (tiles * ksp * kbm * 64 * sizeof(float) > part_cap || tiles > kCounterBytes / sizeof(unsigned))))
+          return fail(QLIN_ERR_UNSUPPORTED, "%s: QLIN_PREFILL_KG=%d,%d unusable here", fn, kbm, ksp);
+        p = PfPlan{true, 0, ksp, 0, kbm};
+      }
+      if (p.kg) {
+        t.splits = p.splits;
+        if (p.splits > 1) {
+          t.cnt = (unsigned*)ws;
+          t.part = (float*)((char*)ws + kPartBase);
+        }
+        return hip_status(fn, launch_prefill_kg(t, wk, zero != nullptr, p.kg, (hipStream_t)stream));
       }
       if (p.tiled || force_tiled) {
         t.splits = p.splits;

@@ -158,6 +158,9 @@ struct TlArgs {
 // wave groups split every K tile's substeps: 4 waves).
 enum PrefillShape { PF_128x128 = 0, PF_256x256 = 1, PF_128x128_K2 = 2, PF_SHAPES = 3 };
 hipError_t launch_prefill(const TlArgs& a, int wk, bool hz, int shape, hipStream_t stream);
+// short-prompt kernel: tiles of bm (32 or 64) rows x 64 columns, a.splits workgroups per tile
+// (partials [tiles][splits][bm * 64]), K % 32 == 0
+hipError_t launch_prefill_kg(const TlArgs& a, int wk, bool hz, int bm, hipStream_t stream);
 // whether the balanced schedule with sk K tiles per workgroup gives every output tile
 // at most two workgroups
 bool prefill_balanced_ok(long long tiles, int nkt, int sk);
