@@ -876,14 +876,9 @@ int engine_gate_up(const char* fn, int wk, int epi, const int8_t* a_q, const flo
   return plan_and_launch(fn, P, a, ws, wsb, (hipStream_t)stream);
 }
 
-// Prefill plan: the LDS-tiled kernel with a tile shape and a split-K factor, or the
-// skinny kernel over row tiles, whichever a time model fitted to MI355X
-// measurements (fp16 x int8, W4 about 1.3x slower per tile) prefers:
-//   tiled:  fixed + rounds x (K tiles per workgroup) x t_tile(workgroups per CU)
-//           + split-K: about 3 us of arrival round trips plus 0.5 us per MB of
-//             partials written and read back
-//   skinny: fixed + cost per (row x MB of int8-sized weights): its 16-row tiles
-//           re-read the weights from L2
+// Prefill plan: the LDS-tiled kernel with a tile shape and a split-K factor or the balanced
+// schedule, the short-prompt kernel, or the skinny kernel over row tiles (its 16-row tiles
+// re-read the weights from L2), whichever a time model fitted to MI355X measurements prefers.
 struct PfPlan {
   bool tiled;
   int shape;
@@ -904,10 +899,11 @@ struct KgTime {
 constexpr KgTime kKgTime[2][2] = {  // [W8, W4][32, 64 rows]
     {{3.8, {0.27, 0.46, 0.73}, 0.0206, 0.36, 0.41, 0.42, 3}, {4.5, {0.30, 0.62, 0}, 0.0243, 0.28, 0.43, 0.37, 2}},
     {{4.0, {0.37, 0.44, 0.65}, 0.0149, 0.11, 0.40, 0.41, 3}, {4.8, {0.46, 0.68, 0}, 0.0133, 0.13, 0.42, 0.41, 2}}};
+// (larger grids were measured behind the large tiles, which re-read less)
 constexpr long long kKgWorkgroups = 1024;
 
 // The best short-prompt plan of a call: its time in seconds (negative if there is none).
-double plan_kg(int wk, int M, int K, int N, size_t part_cap, PfPlan* plan) {
+double plan_kg(int wk, int M, int K, int N, size_t part_cap, long long most, PfPlan* plan) {
   double best = -1.0;
   for (int k = 0; k < 2; ++k) {
     const KgTime& m = kKgTime[wk == WK_W4][k];
@@ -917,7 +913,7 @@ double plan_kg(int wk, int M, int K, int N, size_t part_cap, PfPlan* plan) {
     for (const int S : {1, 2, 3, 4, 6, 8}) {
       const long long wgs = tiles * S;
       const double part = (double)wgs * bm * 64 * sizeof(float);
-      if (wgs > kKgWorkgroups) break;
+      if (wgs > most) break;
       if (S > 1 && (part > (double)part_cap || tiles > (long long)(kCounterBytes / sizeof(unsigned)))) break;
       const int steps = (K / 32 + 4 * S - 1) / (4 * S);
       const long long full = wgs / (256LL * m.cap), rest = wgs - full * 256LL * m.cap;
@@ -930,78 +926,101 @@ double plan_kg(int wk, int M, int K, int N, size_t part_cap, PfPlan* plan) {
   return best;
 }
 
-PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap, bool allow_kg) {
-  // Time model fitted to MI355X measurements with the weights streaming from HBM
-  // (M = 128 / 512 / 2048 on the 2048x6144, 6144x2048 and 2048x2048 shapes):
-  //   tiled:  5 us + rounds x (K tiles per split) x t_tile  (x 1.3 for W4)
-  //           + split-K exchange: 1.45 us per split (the last workgroup reads the
-  //             splits one round trip each) + 12 ns per workgroup + 0.1 us per MB of
-  //             partial tiles; a split level is tried only while the level below it
-  //             leaves CUs idle (split-K exists to fill the chip)
-  //   balanced: 5 us + (K tiles per workgroup) x t_tile + the exchange of the
-  //             tiles shared by two workgroups (below)
-  //   rows:   16-row tiles, 4 waves over the whole K per 128 columns:
-  //           7.1 us (W4 5.8) + max(1, workgroups / 256) x 3.4 ns (W4 2.7) per K row
-  struct Cand {
-    int shape;
-    int per_cu;        // workgroups one CU can hold
-    double t_tile[2];  // seconds per 64-wide K tile of a workgroup, 1 or 2 per CU
-  };
-  const bool w4 = wk == WK_W4;
-  const double w4f = w4 ? 1.3 : 1.0;
-  const Cand cands[2] = {{PF_128x128_K2, 2, {0.48e-6, 1.35e-6}}, {PF_256x256, 1, {1.96e-6, 1.96e-6}}};
+// Time model of the large tiles (prefill_kernel.h), microseconds: t0 + rounds of 256
+// workgroups (one per CU) x 64-wide K tiles x s + the bytes the tiles read, mb per MB + the
+// split-K exchange, xs per split and xmb per MB of partial tiles; the balanced schedule (256x256
+// only) adds bal and runs sk K tiles.  Fitted to MI355X measurements of every shape and split
+// (M = 150-2048, ten shapes from 1024x3072 to 12288x4096): 2-7 % rms, choices 0.6 % from the
+// best on average.  128x384 is for grids that 256x256 leaves short of or just past a round:
+// W8 2048x6144 M = 1300 46.7 us against 52, 4096x12288 M = 700 85.7 against 92.
+struct TiledTime {
+  int shape;
+  double t0, s, mb, xs, xmb, bal;
+};
+constexpr TiledTime kTiledTime[2][3] = {  // W8, W4
+    {{PF_256x256, 6.4, 1.240, 0.0203, 1.90, 0.27, 19.9},
+     {PF_128x128_K2, 5.8, 0.438, 0.0105, 0.65, 0.40, -1},
+     {PF_128x384, 6.6, 1.144, 0.0183, -1, 0, -1}},
+    {{PF_256x256, 6.4, 1.548, 0.0183, 1.96, 0.26, 18.3},
+     {PF_128x128_K2, 6.1, 0.590, 0.0078, 0.66, 0.40, -1},
+     {PF_128x384, 6.7, 1.389, 0.0240, -1, 0, -1}}};
+
+// The best large-tile plan of a call; *t its time in seconds.
+PfPlan plan_tiled(int wk, int M, int K, int N, size_t part_cap, double* t) {
   const int nk = K / 64;
-  PfPlan best{false, PF_128x128_K2, 1, 0, 0};
-  const double row_wgs = (double)((M + 15) / 16) * ((N + 127) / 128);
-  double best_t = (w4 ? 5.8e-6 : 7.1e-6) + (row_wgs > 256 ? row_wgs / 256 : 1.0) * (w4 ? 2.7e-9 : 3.4e-9) * K;
-  for (const Cand& c : cands) {
+  PfPlan best{true, PF_128x128_K2, 1, 0, 0};
+  *t = -1.0;
+  for (const TiledTime& m : kTiledTime[wk == WK_W4]) {
     int bm, bn, waves;
-    prefill_geometry(c.shape, &bm, &bn, &waves);
+    prefill_geometry(m.shape, &bm, &bn, &waves);
     const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const double base = m.t0 + m.mb * 1e-6 * (double)tiles * K * (2.0 * bm + bn * (wk == WK_W4 ? 0.5 : 1.0));
+    const bool counters = tiles <= (long long)(kCounterBytes / sizeof(unsigned));
+    auto take = [&](double us, int S, int sk) {
+      if (*t < 0.0 || us * 1e-6 < *t) *t = us * 1e-6, best = PfPlan{true, m.shape, S, sk, 0};
+    };
     for (int S = 1; S <= 16; S *= 2) {
-      if (nk % S != 0 || nk / S < 2) break;
-      const double part_bytes = (double)tiles * S * waves * 128 * 64 * sizeof(float);
-      if (S > 1 && (part_bytes > (double)part_cap || tiles > (long long)(kCounterBytes / sizeof(unsigned)))) break;
-      const long long wgs = tiles * S;
-      if (S > 1 && tiles * (S / 2) >= 256LL * c.per_cu) break;
-      const int occ = (wgs > 256 && c.per_cu > 1) ? 2 : 1;
-      const double rounds = (double)((wgs + 256LL * occ - 1) / (256LL * occ));
-      const double tile_bytes = (double)wgs * bm * bn * sizeof(float);  // one partial tile per workgroup
-      const double t = 5e-6 + rounds * (nk / S) * c.t_tile[occ - 1] * w4f +
-                       (S > 1 ? 1.45e-6 * S + 12e-9 * wgs + 0.1e-12 * tile_bytes : 0.0);
-      if (t < best_t) {
-        best_t = t;
-        best = PfPlan{true, c.shape, S, 0, 0};
-      }
+      const double part = (double)tiles * S * waves * 128 * 64 * sizeof(float);
+      if (nk % S != 0 || (S > 1 && (nk / S < 2 || m.xs < 0 || part > (double)part_cap || !counters))) break;
+      if (S > 1 && tiles * (S / 2) >= 256) break;  // split-K exists to fill the chip
+      const double rounds = (double)((tiles * S + 255) / 256);
+      take(base + rounds * (nk / S) * m.s +
+               (S > 1 ? m.xs * S + m.xmb * 1e-6 * (double)tiles * S * bm * bn * sizeof(float) : 0.0), S, 0);
     }
-    // Balanced schedule: every CU slot gets the same run of (tile, K tile) units,
-    // crossing tile boundaries.  A tile split over two workgroups moves about 1.8
-    // fp32 partial tiles (one store, two when both pieces end together, and one
-    // load), at about 0.22 us per MB, plus about 2 us for the second piece's
-    // pipeline start (measured, W8 and W4, M = 2048: 2048x6144 in 192 tiles, where
-    // this loses to one tile per workgroup, and 4096x12288 in 384 tiles, where it
-    // wins by 9 %).
-    const long long slots = 256LL * c.per_cu;
-    const long long units = tiles * nk;
-    if (tiles % slots != 0 && tiles > slots / 2 &&
-        tiles <= (long long)(kCounterBytes / sizeof(unsigned)) &&
+    // the balanced schedule: every CU the same run of (tile, K tile) units, across tiles
+    if (m.bal >= 0 && tiles % 256 != 0 && tiles > 128 && counters &&
         (double)tiles * 2 * waves * 128 * 64 * sizeof(float) <= (double)part_cap) {
-      const int sk = (int)((units + slots - 1) / slots);
-      if (prefill_balanced_ok(tiles, nk, sk)) {
-        const int occ = c.per_cu > 1 ? 2 : 1;
-        const double xbytes = 1.8 * (double)tiles * bm * bn * sizeof(float);
-        const double t = 5e-6 + sk * c.t_tile[occ - 1] * w4f + 2e-6 + 0.22e-12 * xbytes;
-        if (t < best_t) {
-          best_t = t;
-          best = PfPlan{true, c.shape, 1, sk, 0};
-        }
-      }
+      const int sk = (int)((tiles * nk + 255) / 256);
+      if (prefill_balanced_ok(tiles, nk, sk)) take(base + m.bal + sk * m.s, 1, sk);
     }
   }
-  // the short-prompt kernel, where its model is 10 % ahead (the models above are off by
-  // about that much): 2048x2048 at M = 128 13.6 -> 8.1 us (W8), 6144x2048 21.5 -> 13.3 (W4)
+  return best;
+}
+
+// Whether a W4 call may use the large tiles: they round the group scales into the fp16
+// weights, where the 16-row tiles and the short-prompt kernel multiply fp32 dots by them, so
+// calls on the 16-row tiles' side of this line (their time against tiles of 128x128 and
+// 256x256, microseconds) keep the fp32 form.
+bool w4_large_tiles(int M, int K, int N, size_t part_cap) {
+  const double row_wgs = (double)((M + 15) / 16) * ((N + 127) / 128);
+  const double t_rows = 5.8 + std::max(1.0, row_wgs / 256) * 2.7e-3 * K;
+  const int nk = K / 64;
+  for (const int big : {0, 1}) {
+    const int b = big ? 256 : 128, per_cu = big ? 1 : 2, waves = big ? 8 : 4;
+    const long long tiles = (long long)((M + b - 1) / b) * ((N + b - 1) / b);
+    for (int S = 1; S <= 16; S *= 2) {
+      if (nk % S != 0 || nk / S < 2) break;
+      if (S > 1 && ((double)tiles * S * waves * 128 * 64 * sizeof(float) > (double)part_cap ||
+                    tiles > (long long)(kCounterBytes / sizeof(unsigned)) || tiles * (S / 2) >= 256LL * per_cu))
+        break;
+      const long long wgs = tiles * S;
+      const int occ = (wgs > 256 && per_cu > 1) ? 2 : 1;
+      const double t_tile = big ? 1.96 : (occ == 2 ? 1.35 : 0.48);
+      const double t = 5.0 + (double)((wgs + 256LL * occ - 1) / (256LL * occ)) * (nk / S) * t_tile * 1.3 +
+                       (S > 1 ? 1.45 * S + 0.012 * wgs + 0.1e-6 * (double)wgs * b * b * sizeof(float) : 0.0);
+      if (t < t_rows) return true;
+    }
+  }
+  return false;
+}
+
+PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap, bool force_tiled) {
+  // rows: 16-row tiles, 4 waves over the whole K per 128 columns, 7.1 us (W4 5.8) + max(1,
+  // workgroups / 256) x 3.4 ns (W4 2.7) per K row
+  const bool w4 = wk == WK_W4;
+  const double row_wgs = (double)((M + 15) / 16) * ((N + 127) / 128);
+  const double t_rows = (w4 ? 5.8e-6 : 7.1e-6) + std::max(1.0, row_wgs / 256) * (w4 ? 2.7e-9 : 3.4e-9) * K;
+  double t_tiled = 0.0;
+  const PfPlan tiled = plan_tiled(wk, M, K, N, part_cap, &t_tiled);
+  if (force_tiled) return tiled;
+  PfPlan best{false, PF_128x128_K2, 1, 0, 0};
+  double best_t = t_rows;
+  const bool large = !w4 || w4_large_tiles(M, K, N, part_cap);
+  if (large && t_tiled < best_t) best = tiled, best_t = t_tiled;
+  // the short-prompt kernel, where its model is 10 % ahead (the rows model is off by about
+  // that much): 2048x2048 at M = 128 13.6 -> 8.1 us (W8), 6144x2048 21.5 -> 13.3 (W4)
   PfPlan kg;
-  const double t_kg = allow_kg ? plan_kg(wk, M, K, N, part_cap, &kg) : -1.0;
+  const double t_kg = plan_kg(wk, M, K, N, part_cap, large ? kKgWorkgroups : 1LL << 20, &kg);
   if (t_kg >= 0.0 && t_kg < 0.9 * best_t) return kg;
   return best;
 }
@@ -1082,7 +1101,7 @@ int a16_linear(const char* fn, int wk, const void* x, int x_dtype, int M, int K,
     t.sk = 0;
     t.gm = 0;
     if (fits32) {
-      PfPlan p = plan_prefill(wk, M, K, N, part_cap, !force_tiled);
+      PfPlan p = plan_prefill(wk, M, K, N, part_cap, force_tiled);
       if (getenv("QLIN_PREFILL_VERBOSE"))
         fprintf(stderr, "qlin prefill plan M=%d K=%d N=%d: %s shape=%d splits=%d sk=%d\n", M, K, N,
                 p.kg ? "short" : p.tiled ? "tiled" : "skinny", p.kg ? p.kg : p.shape, p.splits, p.sk);

@@ -9,8 +9,10 @@ void prefill_geometry(int shape, int* bm, int* bn, int* waves) {
   using G0 = Geo<WK_W8, 1, 2, 1>;
   using G1 = Geo<WK_W8, 2, 4, 1>;
   using G2 = Geo<WK_W8, 1, 2, 2>;
+  using G3 = Geo<WK_W8, 2, 6, 1, 3, 4>;
   if (shape == PF_128x128) *bm = G0::BM, *bn = G0::BN, *waves = G0::WAVES;
   else if (shape == PF_128x128_K2) *bm = G2::BM, *bn = G2::BN, *waves = G2::WAVES;
+  else if (shape == PF_128x384) *bm = G3::BM, *bn = G3::BN, *waves = G3::WAVES;
   else *bm = G1::BM, *bn = G1::BN, *waves = G1::WAVES;
 }
 

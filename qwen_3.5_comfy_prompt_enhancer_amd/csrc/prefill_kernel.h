@@ -6,9 +6,12 @@
 // [K,N] with per-column scales, or packed nibbles [K/2,N] with per-group scales and
 // optional zeros).
 //
-//   * Workgroup tile BM x BN = (128 WM) x (64 WN) computed by WM x WN waves, each
-//     owning a 128 x 64 output tile = 8 x 4 blocks of v_mfma_f32_16x16x32_f16 with
-//     fp32 accumulation.  Tall wave tiles make every dequantized weight operand feed
+//   * Workgroup tile BM x BN = (16 RW WM) x (64 WN) computed by WM x WN waves, each
+//     owning a 16 RW x 64 output tile = RW x 4 blocks of v_mfma_f32_16x16x32_f16 with
+//     fp32 accumulation; RW = 8 but for the 128 x 384 tile (12 waves of 64 x 64, three per
+//     SIMD), whose area is three quarters of 256 x 256 for grids that the larger tile leaves
+//     just past a round (it reads more LDS bytes per MFMA: the same time per tile and K step,
+//     1.15-1.25 us, less the rows and columns it saves).  Tall wave tiles make every dequantized weight operand feed
 //     8 MFMAs.  With 8 waves (256 x 256) two waves share each SIMD, so one wave's
 //     dequantization and LDS traffic issue while the other's MFMAs run.  With KG = 2
 //     wave groups, each group computes one of the two 32-wide substeps of every K
@@ -61,10 +64,10 @@ namespace {
 constexpr int BK = 64;           // K per stage
 constexpr int GROUP_M = 8;       // tile order: 8 row tiles per group
 
-template <int WK, int WM, int WN, int KG, int NS = 3>
+template <int WK, int WM, int WN, int KG, int NS = 3, int RW = 8>
 struct Geo {
   static constexpr int NSTAGE = NS;  // K tiles in the LDS ring
-  static constexpr int BM = 128 * WM;
+  static constexpr int BM = 16 * RW * WM;  // RW 16-row blocks per wave
   static constexpr int BN = 64 * WN;  // WN even: the weight tile is stored in 128-column halves
   static constexpr int WAVES = WM * WN * KG;  // KG wave groups split each K tile's substeps
   static constexpr int THREADS = 64 * WAVES;
@@ -79,13 +82,22 @@ struct Geo {
   static constexpr int B_BYTES = B_BLOCKS * WB;
   static constexpr int SC_BYTES = (WK == WK_W8) ? 0 : WAVES * 1024;  // W4 scales + zeros
   static constexpr int STAGE = A_BYTES + B_BYTES + SC_BYTES;
-  static constexpr int A_DMA = (BM / 8) / WAVES;  // 1 KB activation blocks per wave
+  static constexpr int A_BLOCKS = BM / 8;  // 1 KB activation blocks; block q of a wave is a_block(wave, q)
+  static constexpr int A_DMA = (A_BLOCKS + WAVES - 1) / WAVES;
+  // (where they do not divide evenly, a wave past the last block copies its first one again,
+  // so every wave waits for the same number of copies)
+  static __device__ __forceinline__ int a_block(int wave, int q) {
+    if constexpr (A_BLOCKS % WAVES == 0) return wave * A_DMA + q;
+    const int b = wave + WAVES * q;
+    return b < A_BLOCKS ? b : wave;
+  }
   static constexpr int B_DMA = B_BLOCKS / WAVES;  // weight blocks per wave
   static constexpr int DMA = A_DMA + B_DMA + (WK == WK_W4 ? 1 : 0);  // copies per wave per stage
-  static constexpr int OCC = (WAVES >= 8) ? 2 : 1;                    // waves per SIMD
-  static_assert(WN % 2 == 0 && (BM / 8) % WAVES == 0 && B_BLOCKS % WAVES == 0, "tile geometry");
+  static constexpr int OCC = (WAVES + 3) / 4 > 3 ? 3 : (WAVES >= 8) ? WAVES / 4 : 1;  // waves per SIMD
+  static_assert(WN % 2 == 0 && A_DMA <= 2 * (A_BLOCKS / WAVES) && B_BLOCKS % WAVES == 0, "tile geometry");
+  static constexpr int WT = 16 * RW * 64;  // outputs of a wave
   static_assert(KG == 1 || KG == 2, "one or two K groups");
-  static_assert(KG == 1 || NSTAGE * STAGE >= WM * WN * 128 * 64 * 4, "LDS for the K-group reduction");
+  static_assert(KG == 1 || NSTAGE * STAGE >= WM * WN * WT * 4, "LDS for the K-group reduction");
   static_assert(WK == WK_W8 || 10 * BN <= SC_BYTES, "W4 scale region");
 };
 
@@ -138,11 +150,11 @@ __device__ __forceinline__ _Float16 scale_f16(const uint32_t (&w)[4], int t) {
 
 // SD: the W4 scale dtype (DT_F16, DT_BF16 or DT_F32); 0 for W8, whose column scales
 // are read once per tile, in the epilogue, in any dtype.
-template <int WK, bool HZ, int SD, int WM, int WN, int KG, int NS, bool BAL>
+template <int WK, bool HZ, int SD, int WM, int WN, int KG, int NS, int RW, bool BAL>
 __global__ __launch_bounds__(64 * WM * WN * KG)
-__attribute__((amdgpu_waves_per_eu(Geo<WK, WM, WN, KG, NS>::OCC, Geo<WK, WM, WN, KG, NS>::OCC)))
+__attribute__((amdgpu_waves_per_eu(Geo<WK, WM, WN, KG, NS, RW>::OCC, Geo<WK, WM, WN, KG, NS, RW>::OCC)))
 void prefill_kernel(const TlArgs a) {
-  using G = Geo<WK, WM, WN, KG, NS>;
+  using G = Geo<WK, WM, WN, KG, NS, RW>;
   constexpr int NSTAGE = G::NSTAGE;
   constexpr int BN = G::BN;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -187,7 +199,7 @@ void prefill_kernel(const TlArgs a) {
   uint32_t offA[G::A_DMA];
 #pragma unroll
   for (int q = 0; q < G::A_DMA; ++q) {
-    const int r = 8 * (wave * G::A_DMA + q) + (lane >> 3);
+    const int r = 8 * G::a_block(wave, q) + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     const int row = min(m0 + r, M - 1);  // rows past M read row M-1 and are never stored
     offA[q] = (uint32_t)(((long long)row * a.ldx + 8 * c) * 2);
@@ -237,7 +249,7 @@ void prefill_kernel(const TlArgs a) {
     const uint32_t base = lds0 + (uint32_t)(st * G::STAGE);
     const void* xa = rfl_ptr(a.x + k0);
 #pragma unroll
-    for (int q = 0; q < G::A_DMA; ++q) dma_s(xa, offA[q], rfl(base + (uint32_t)((wave * G::A_DMA + q) * 1024)));
+    for (int q = 0; q < G::A_DMA; ++q) dma_s(xa, offA[q], rfl(base + (uint32_t)(G::a_block(wave, q) * 1024)));
     const void* wb = rfl_ptr(a.w + (long long)((WK == WK_W8) ? k0 : k0 / 2) * N);
 #pragma unroll
     for (int q = 0; q < G::B_DMA; ++q)
@@ -264,16 +276,16 @@ void prefill_kernel(const TlArgs a) {
     }
   };
 
-  f32x4 acc[8][4];
+  f32x4 acc[RW][4];
 #pragma unroll
-  for (int rb = 0; rb < 8; ++rb)
+  for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[rb][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Operands of one 32-wide K substep: 8 activation blocks, the raw weight dwords
+  // Operands of one 32-wide K substep: RW activation blocks, the raw weight dwords
   // (8 int8 rows or 4 packed rows of 4 columns) and, for W4, 4 scales and 4 zeros.
   struct Ops {
-    f16x8 av[8];
+    f16x8 av[RW];
     uint32_t d[8];
     uint32_t sv[4];
     uint32_t zv;
@@ -297,8 +309,8 @@ void prefill_kernel(const TlArgs a) {
     const uint8_t* sB = sA + G::A_BYTES;
     const uint8_t* sS = sB + G::B_BYTES;
 #pragma unroll
-    for (int rb = 0; rb < 8; ++rb) {
-      const int row = wm * 128 + rb * 16 + j;
+    for (int rb = 0; rb < RW; ++rb) {
+      const int row = wm * 16 * RW + rb * 16 + j;
       o.av[rb] = *(const f16x8*)(sA + row * 128 + 16 * ((4 * ks + g) ^ (j >> 1)));
     }
     if constexpr (WK == WK_W8) {
@@ -338,14 +350,14 @@ void prefill_kernel(const TlArgs a) {
     return bitcast<f16x8>(h);
   };
 
-  // column-outer order: the dequantization of column t + 1 overlaps the 8 MFMAs of
+  // column-outer order: the dequantization of column t + 1 overlaps the RW MFMAs of
   // column t
   auto mma = [&](const Ops& o) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const f16x8 bv = dequant(o, t);
 #pragma unroll
-      for (int rb = 0; rb < 8; ++rb) acc[rb][t] = mfma_f16(o.av[rb], bv, acc[rb][t]);
+      for (int rb = 0; rb < RW; ++rb) acc[rb][t] = mfma_f16(o.av[rb], bv, acc[rb][t]);
     }
   };
 
@@ -361,7 +373,7 @@ void prefill_kernel(const TlArgs a) {
     // and two VALU slots
     __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);  // VALU
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < 4 * RW; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
       __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
@@ -392,7 +404,7 @@ void prefill_kernel(const TlArgs a) {
       __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);  // DS reads
       __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);  // VALU
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
+      for (int i = 0; i < 4 * RW; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
         __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
       }
@@ -443,11 +455,11 @@ void prefill_kernel(const TlArgs a) {
   if constexpr (KG == 2) {
     // K-group reduction through the (now idle) LDS stages: group 1 writes its
     // accumulators, group 0 adds them (fixed order: group 0 + group 1)
-    float* red = (float*)lds + (long long)wl * (128 * 64) + lane;
+    float* red = (float*)lds + (long long)wl * G::WT + lane;
     asm volatile("s_barrier" ::: "memory");  // every wave's last LDS read has returned
     if (kg == 1) {
 #pragma unroll
-      for (int rb = 0; rb < 8; ++rb)
+      for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -456,7 +468,7 @@ void prefill_kernel(const TlArgs a) {
     __syncthreads();
     if (kg == 0) {
 #pragma unroll
-      for (int rb = 0; rb < 8; ++rb)
+      for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -469,15 +481,15 @@ void prefill_kernel(const TlArgs a) {
     // ((rb * 4 + t) * 64 + lane) * 16 of the wave's slot, so each store or load
     // instruction moves 1 KiB contiguous.  Device-coherent (SC1) stores and loads;
     // each workgroup's stores complete before it signals.
-    constexpr unsigned kSlot = 128u * 64u * 4u;  // bytes of one wave's partial tile
+    constexpr unsigned kSlot = G::WT * 4u;  // bytes of one wave's partial tile
     const __amdgpu_buffer_rsrc_t rs =
-        part_rsrc(a.part + (long long)tile * xs * G::WAVES * (128 * 64), (unsigned)(xs * G::WAVES) * kSlot);
+        part_rsrc(a.part + (long long)tile * xs * G::WAVES * G::WT, (unsigned)(xs * G::WAVES) * kSlot);
     const unsigned lane_off = (unsigned)lane * 16u;
     auto store_partial = [&]() {
       if (kg == 0) {
         const unsigned base = (unsigned)(xslot * G::WAVES + wl) * kSlot + lane_off;
 #pragma unroll
-        for (int rb = 0; rb < 8; ++rb)
+        for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
           for (int t = 0; t < 4; ++t) st_coherent(acc[rb][t], rs, base + (unsigned)(rb * 4 + t) * 1024u);
       }
@@ -501,7 +513,7 @@ void prefill_kernel(const TlArgs a) {
       for (int sp = 0; sp < xs; ++sp) {
         const unsigned base = (unsigned)(sp * G::WAVES + wl) * kSlot + lane_off;
 #pragma unroll
-        for (int rb = 0; rb < 8; ++rb)
+        for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             const f32x4 v = ld_coherent(rs, base + (unsigned)(rb * 4 + t) * 1024u);
@@ -534,7 +546,7 @@ void prefill_kernel(const TlArgs a) {
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       const unsigned base = (unsigned)((1 - xslot) * G::WAVES + wl) * kSlot + lane_off;
 #pragma unroll
-      for (int rb = 0; rb < 8; ++rb)
+      for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[rb][t] = acc[rb][t] + ld_coherent(rs, base + (unsigned)(rb * 4 + t) * 1024u);
     }
@@ -550,8 +562,8 @@ void prefill_kernel(const TlArgs a) {
   // 128 values of a lane costs a multiply, a conversion and (with a residual) an add.
   // Row addresses are a uniform base (the wave's first row) plus a per-lane offset
   // computed once, plus a uniform multiple of the row stride.
-  const int r0 = m0 + wm * 128;       // first row of the wave
-  const int nrows = M - r0;           // rows of the wave below M (may exceed 128)
+  const int r0 = m0 + wm * 16 * RW;   // first row of the wave
+  const int nrows = M - r0;           // rows of the wave below M (may exceed its own)
   uint16_t* const obase = (uint16_t*)a.out + (long long)r0 * a.ldo;
   const uint16_t* const rbase = a.res ? (const uint16_t*)a.res + (long long)r0 * a.ldr : nullptr;
   const long long oofs = (long long)(4 * g) * a.ldo + colb, rofs = (long long)(4 * g) * a.ldr + colb;
@@ -563,7 +575,7 @@ void prefill_kernel(const TlArgs a) {
       else return bitcast<uint32_t>(__builtin_convertvector((float __attribute__((ext_vector_type(2)))){v0, v1}, f16x2));
     };
 #pragma unroll
-    for (int rb = 0; rb < 8; ++rb)
+    for (int rb = 0; rb < RW; ++rb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (rb * 16 + 4 * g + r >= nrows) continue;
@@ -630,21 +642,21 @@ void prefill_kernel(const TlArgs a) {
   }
 }
 
-template <int WK, bool HZ, int SD, int WM, int WN, int KG, int NS, bool BAL>
+template <int WK, bool HZ, int SD, int WM, int WN, int KG, int NS, bool BAL, int RW = 8>
 static hipError_t launch_prefill_t(const TlArgs& a, hipStream_t st) {
-  using G = Geo<WK, WM, WN, KG, NS>;
+  using G = Geo<WK, WM, WN, KG, NS, RW>;
   const long long tiles = (long long)((a.M + G::BM - 1) / G::BM) * ((a.N + G::BN - 1) / G::BN);
   const long long units = tiles * (a.K / BK);
   const int wgs = (int)(a.sk > 0 ? (units + a.sk - 1) / a.sk : tiles * a.splits);
   const size_t lds = (size_t)G::NSTAGE * G::STAGE;
   static bool attr_set = false;  // benign race: every caller sets the same value
   if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute((const void*)prefill_kernel<WK, HZ, SD, WM, WN, KG, NS, BAL>,
+    const hipError_t e = hipFuncSetAttribute((const void*)prefill_kernel<WK, HZ, SD, WM, WN, KG, NS, RW, BAL>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
-  hipLaunchKernelGGL((prefill_kernel<WK, HZ, SD, WM, WN, KG, NS, BAL>), dim3(wgs), dim3(G::THREADS), lds, st, a);
+  hipLaunchKernelGGL((prefill_kernel<WK, HZ, SD, WM, WN, KG, NS, RW, BAL>), dim3(wgs), dim3(G::THREADS), lds, st, a);
   return hipGetLastError();
 }
 
@@ -661,6 +673,8 @@ static hipError_t launch_prefill_kind(const TlArgs& a, int shape, hipStream_t st
       return bal ? launch_prefill_t<WK, HZ, SD, 1, 2, 2, 3, true>(a, st) : launch_prefill_t<WK, HZ, SD, 1, 2, 2, 3, false>(a, st);
     case PF_256x256:
       return bal ? launch_prefill_t<WK, HZ, SD, 2, 4, 1, 3, true>(a, st) : launch_prefill_t<WK, HZ, SD, 2, 4, 1, 3, false>(a, st);
+    case PF_128x384:  // one tile per workgroup only (no balanced schedule)
+      return bal ? hipErrorInvalidValue : launch_prefill_t<WK, HZ, SD, 2, 6, 1, 3, false, 4>(a, st);
     default:
       return hipErrorInvalidValue;
   }

@@ -154,9 +154,10 @@ struct TlArgs {
 };
 
 // LDS-DMA prefill kernel; `shape` picks the workgroup tile (rows x columns):
-// PF_128x128 (2 waves), PF_256x256 (8 waves, two per SIMD) and PF_128x128_K2 (two
-// wave groups split every K tile's substeps: 4 waves).
-enum PrefillShape { PF_128x128 = 0, PF_256x256 = 1, PF_128x128_K2 = 2, PF_SHAPES = 3 };
+// PF_128x128 (2 waves), PF_256x256 (8 waves, two per SIMD), PF_128x128_K2 (two
+// wave groups split every K tile's substeps: 4 waves), PF_128x384 (12 waves of 64 x 64, three
+// per SIMD).
+enum PrefillShape { PF_128x128 = 0, PF_256x256 = 1, PF_128x128_K2 = 2, PF_128x384 = 3, PF_SHAPES = 4 };
 hipError_t launch_prefill(const TlArgs& a, int wk, bool hz, int shape, hipStream_t stream);
 // short-prompt kernel: tiles of bm (32 or 64) rows x 64 columns, a.splits workgroups per tile
 // (partials [tiles][splits][bm * 64]), K % 32 == 0

@@ -73,3 +73,24 @@ def test_graph_replays():
         g.replay()
         assert torch.equal(o, eager)
         assert torch.equal(linear.linear_w8(x, w, s, torch.empty_like(o)), eager)
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 512, 64), (129, 64, 400), (300, 1024, 1280)])
+def test_wide_tile(monkeypatch, M, K, N):
+    """The 128 x 384 tile of the large-tile kernel (QLIN_PREFILL_SHAPE=3): the bits of the
+    256 x 256 tile (one K order), W8 with a residual and W4 with zeros in each scale dtype."""
+    from qwen35_amd.kernels import linear
+    x = H.act_f16(M, K, seed=M).cuda()
+    w, s = (t.cuda() for t in H.w8(K, N, seed=N))
+    p, s4, z = (t.cuda() for t in H.w4(K, N, seed=N, group=32, zeros="random"))
+    res = torch.randn((M, N), generator=H.gen(9)).to(torch.float16).cuda()
+    monkeypatch.setenv("QLIN_PREFILL", "tiled")
+    outs = []
+    for shape in (1, 3):
+        monkeypatch.setenv("QLIN_PREFILL_SHAPE", str(shape))
+        o = [linear.linear_w8(x, w, s, torch.empty_like(res), residual=res)]
+        for dt in (torch.float16, torch.bfloat16, torch.float32):
+            o.append(linear.linear_w4(x, p, s4.to(dt), torch.empty_like(res), w_zero=z))
+        outs.append(o)
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    H.assert_out_close(outs[1][0], H.linear_w8_ref_cols(x.cpu(), w.cpu(), s.cpu(), np.arange(N), residual=res.cpu()))
