@@ -18,8 +18,10 @@
 //     chip half idle: with 137 rows the 128-row tile computes 256.  The host's time model
 //     (abi.hip, tile_time) chooses; the K order and so the bits are the same.  A stage of
 //     the LDS ring holds two activation blocks (128 K); group kg computes block
-//     2 * stage + kg, and at the end group 1's accumulators are added to group 0's through
-//     LDS (fixed order).
+//     2 * stage + kg; at the end the two groups' accumulators are added through LDS, each
+//     group finishing half of the 16-row blocks (group 0 finishing all of them left four of
+//     eight waves idle in the epilogue: a W8 2048-hidden layer's linears at M = 512 134.2 ->
+//     131.6 us with the producers, a W4 4096-hidden one's at M = 137 220.9 -> 216.7).
 //   * MFMA: v_mfma_i32_16x16x64_i8, one instruction per 64-wide block, started from
 //     an inline zero, with the weights as its A operand and the activations as B: lane
 //     (g, j) supplies K bytes 16g..16g+15 of weight column 4j + t and of activation row j,
@@ -462,32 +464,37 @@ void prefill_i8_kernel(const SkArgs a) {
       csraw[s][r] = W4 ? u32x4{0u, 0u, 0u, 0u} : ld_scale4_raw(sset[s], a.sdt, ncol0 + ccol + 4 * r);
 
   // ---------------- K groups: group 0 + group 1 (fixed order), one set at a time ----------------
+  // Each group finishes half of the 16-row blocks: it takes the other's sums of them (the two
+  // are added either way round to the same bits) and runs their epilogue, so no wave sits out
+  // the epilogue's divisions and exponentials.
   constexpr int WT = 2 * WNW;  // wave tiles (wm, wn) of one K group
+  constexpr int RH = (RB + 1) / 2;
+  auto mine = [&](int rb) { return (rb < RH) == (kg == 0); };
   const int wt = wave % WT;
   float* red = (float*)lds + wt * (16 * RB * 64) + lane;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    if (s > 0) __syncthreads();  // group 0 has read the previous set
-    if (kg == 1) {
+    if (s > 0) __syncthreads();  // the previous set has been read
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+    for (int rb = 0; rb < RB; ++rb) {
+      if (mine(rb)) continue;  // uniform over a wave
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) red[((rb * 4 + t) * 4 + r) * 64] = acc[s][rb][t][r];
+        for (int r = 0; r < 4; ++r) red[((rb * 4 + t) * 4 + r) * 64] = acc[s][rb][t][r];
     }
     __syncthreads();
-    if (kg == 0) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+    for (int rb = 0; rb < RB; ++rb) {
+      if (!mine(rb)) continue;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[s][rb][t][r] += red[((rb * 4 + t) * 4 + r) * 64];
+        for (int r = 0; r < 4; ++r) acc[s][rb][t][r] += red[((rb * 4 + t) * 4 + r) * 64];
     }
   }
   if (S > 1) {
-    // Split-K: group 0's partial tile of each weight set (wave w: the float4 (rb, t) of
+    // Split-K: the partial tile of each weight set (wave tile w: the float4 (rb, t) of
     // every lane at byte ((rb * 4 + t) * 64 + lane) * 16 of its slot, slots
     // [split][set][wave]) goes out through device-coherent stores; each workgroup's
     // stores complete before it counts its arrival, and the last to arrive sums the
@@ -497,14 +504,14 @@ void prefill_i8_kernel(const SkArgs a) {
     const __amdgpu_buffer_rsrc_t rs =
         part_rsrc(a.part + (long long)tile * S * NS * WT * (16 * RB * 64), (unsigned)(S * NS * WT) * kSlot);
     const unsigned lane_off = (unsigned)lane * 16u;
-    if (kg == 0) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const unsigned base = (unsigned)((split * NS + s) * WT + wt) * kSlot + lane_off;
+    for (int s = 0; s < NS; ++s) {
+      const unsigned base = (unsigned)((split * NS + s) * WT + wt) * kSlot + lane_off;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RB; ++rb) {
+        if (!mine(rb)) continue;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) st_coherent(acc[s][rb][t], rs, base + (unsigned)(rb * 4 + t) * 1024u);
+        for (int t = 0; t < 4; ++t) st_coherent(acc[s][rb][t], rs, base + (unsigned)(rb * 4 + t) * 1024u);
       }
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -518,23 +525,24 @@ void prefill_i8_kernel(const SkArgs a) {
       s_last = last;
     }
     __syncthreads();
-    if (!s_last || kg != 0) return;  // uniform over each wave
+    if (!s_last) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     for (int sp = 0; sp < S; ++sp) {
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const unsigned base = (unsigned)((sp * NS + s) * WT + wt) * kSlot + lane_off;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RB; ++rb) {
+          if (!mine(rb)) continue;
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             const f32x4 v = ld_coherent(rs, base + (unsigned)(rb * 4 + t) * 1024u);
             acc[s][rb][t] = (sp == 0) ? v : acc[s][rb][t] + v;
           }
+        }
       }
     }
   }
-  if (kg != 0) return;
 
   // ---------------- epilogue ----------------
   // Lane (g, j): columns 16g .. 16g + 15 of the wave's 64 (column 4r + t of them in
@@ -562,7 +570,7 @@ void prefill_i8_kernel(const SkArgs a) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int row = r0 + rb * 16;
-        if (row >= M) continue;
+        if (!mine(rb) || row >= M) continue;
         uint16_t* const o = (uint16_t*)a.out + (long long)row * a.ldo + ocol;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -600,6 +608,7 @@ void prefill_i8_kernel(const SkArgs a) {
     // each): the amax reduces over those lanes.
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
+      if (!mine(rb)) continue;
       const int row = r0 + rb * 16;
       float h[16];
 #pragma unroll
