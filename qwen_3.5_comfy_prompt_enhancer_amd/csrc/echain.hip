@@ -682,12 +682,15 @@ __device__ __forceinline__ bool unit_finish(const EJob& J, const EPos& P, int M,
         am = fmaxf(am, fabsf(h[e]));
       }
       if (!valid) am = 0.0f;
-#pragma unroll
-      for (int m = 1; m < 16; m <<= 1) am = fmaxf(am, __shfl_xor(am, m));
+      am = fmaxf(am, lane_xor<1>(am));
+      am = fmaxf(am, lane_xor<2>(am));
+      am = fmaxf(am, lane_xor<4>(am));
+      am = fmaxf(am, lane_xor<8>(am));
       const float sc = fmaxf(am / 127.0f, 1e-8f);
+      const float inv = 1.0f / sc;
       uint32_t qw = 0u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) qw |= ((uint32_t)round_i8(h[e] / sc) & 0xFFu) << (8 * e);
+      for (int e = 0; e < 4; ++e) qw |= ((uint32_t)quant_i8(h[e], sc, inv) & 0xFFu) << (8 * e);
       if (valid) {
         const __amdgpu_buffer_rsrc_t qr = part_rsrc(J.oq, (unsigned)((long long)M * N));
         __builtin_amdgcn_raw_buffer_store_b32(qw, qr, (unsigned)((long long)row * N + gc), 0, kCpolSc1);

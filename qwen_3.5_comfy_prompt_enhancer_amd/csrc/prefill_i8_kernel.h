@@ -631,16 +631,18 @@ void prefill_i8_kernel(const SkArgs a) {
           h[c] = bf16_to_f32(f32_to_bf16(h[c]));  // bf16 round trip (kernels/gemm.py:198-200)
           am = fmaxf(am, fabsf(h[c]));
         }
-        am = fmaxf(am, __shfl_xor(am, 16));
-        am = fmaxf(am, __shfl_xor(am, 32));
-        const float sc = fmaxf(am / 127.0f, 1e-8f);
+        float am0, am1;
+        lane_pair<16>(am, am0, am1);
+        lane_pair<32>(fmaxf(am0, am1), am0, am1);
+        const float sc = fmaxf(fmaxf(am0, am1) / 127.0f, 1e-8f);
+        const float inv = 1.0f / sc;
         if (row < M) {
           uint32_t qw[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             qw[q] = 0;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) qw[q] |= ((uint32_t)(round_i8(h[4 * q + t] / sc) & 0xFF)) << (8 * t);
+            for (int t = 0; t < 4; ++t) qw[q] |= ((uint32_t)(quant_i8(h[4 * q + t], sc, inv) & 0xFF)) << (8 * t);
           }
           *(u32x4*)(a.oq + (long long)row * a.ncols + col) = u32x4{qw[0], qw[1], qw[2], qw[3]};
           if (g == 0) a.os[(long long)row * (a.ncols / 64) + col / 64] = sc;

@@ -63,7 +63,20 @@ __device__ __forceinline__ float pro_rms_inv(float ss, int n, float eps) {
 // every lane of the team ends with the same value.
 __device__ __forceinline__ float pro_team_sum(float acc, int lanes) {
 #pragma clang fp contract(off)
-  for (int m = lanes >> 1; m >= 1; m >>= 1) acc = acc + __shfl_xor(acc, m);
+  if (lanes >= 64) {
+    float a, b;
+    lane_pair<32>(acc, a, b);
+    acc = a + b;
+  }
+  if (lanes >= 32) {
+    float a, b;
+    lane_pair<16>(acc, a, b);
+    acc = a + b;
+  }
+  if (lanes >= 16) acc = acc + lane_xor<8>(acc);
+  if (lanes >= 8) acc = acc + lane_xor<4>(acc);
+  if (lanes >= 4) acc = acc + lane_xor<2>(acc);
+  if (lanes >= 2) acc = acc + lane_xor<1>(acc);
   return acc;
 }
 
@@ -73,13 +86,14 @@ __device__ __forceinline__ float pro_quant8(const float y[8], uint32_t& lo, uint
   float am = 0.0f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(y[e]));
-  am = fmaxf(am, __shfl_xor(am, 1));
-  am = fmaxf(am, __shfl_xor(am, 2));
-  am = fmaxf(am, __shfl_xor(am, 4));
+  am = fmaxf(am, lane_xor<1>(am));
+  am = fmaxf(am, lane_xor<2>(am));
+  am = fmaxf(am, lane_xor<4>(am));
   const float s = fmaxf(am / 127.0f, 1e-8f);
+  const float inv = 1.0f / s;
   uint32_t w[2] = {0u, 0u};
 #pragma unroll
-  for (int e = 0; e < 8; ++e) w[e >> 2] |= ((uint32_t)round_i8(y[e] / s) & 0xFFu) << (8 * (e & 3));
+  for (int e = 0; e < 8; ++e) w[e >> 2] |= ((uint32_t)quant_i8(y[e], s, inv) & 0xFFu) << (8 * (e & 3));
   lo = w[0];
   hi = w[1];
   return s;

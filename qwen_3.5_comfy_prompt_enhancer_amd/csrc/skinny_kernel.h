@@ -827,12 +827,14 @@ __attribute__((amdgpu_waves_per_eu(SkOcc<ACT, WK, EPI, COLS>::value))) void skin
           am = fmaxf(am, fabsf(h[e]));
         }
         if (!cval) am = 0.0f;
-#pragma unroll
-        for (int m = 1; m < 8; m <<= 1) am = fmaxf(am, __shfl_xor(am, m));
+        am = fmaxf(am, lane_xor<1>(am));
+        am = fmaxf(am, lane_xor<2>(am));
+        am = fmaxf(am, lane_xor<4>(am));
         const float sc = fmaxf(am / 127.0f, 1e-8f);
+        const float inv = 1.0f / sc;
         int q[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) q[e] = round_i8(h[e] / sc);
+        for (int e = 0; e < 8; ++e) q[e] = quant_i8(h[e], sc, inv);
         if (cval) {
           st_i8<8>(a.oq + (long long)orow * a.ncols + oc, q);
           if ((c & 63) == 0) a.os[(long long)orow * (a.ncols / 64) + oc / 64] = sc;
