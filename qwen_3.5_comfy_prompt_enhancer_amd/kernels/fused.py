@@ -159,18 +159,16 @@ def pro_gemm_i8(pro: Producer, b, b_s, out, residual=None, b_z=None):
     if residual is not None:
         _check_out("residual", residual, M, N)
     C.require_cuda(*pro.tensors(), b, b_s, b_z, out, residual)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     p = pro.c_struct()
     ldr = residual.stride(0) if residual is not None else 0
     if _is_w4(b):
         st = _fn("qlin_pro_gemm_w4")(ctypes.byref(p), M, K, C.ptr(b), C.ptr(b_s), C.dtype_code(b_s), C.ptr(b_z),
-                                     grp, N, C.ptr(out), out.stride(0), C.ptr(residual), ldr, C.ptr(ws),
-                                     ws.numel(), C.stream_of(out))
+                                     grp, N, C.ptr(out), out.stride(0), C.ptr(residual), ldr, ws, wsb, stream)
         C.check(st, "qlin_pro_gemm_w4")
     else:
         st = _fn("qlin_pro_gemm_i8")(ctypes.byref(p), M, K, C.ptr(b), C.ptr(b_s), C.dtype_code(b_s), N,
-                                     C.ptr(out), out.stride(0), C.ptr(residual), ldr, C.ptr(ws), ws.numel(),
-                                     C.stream_of(out))
+                                     C.ptr(out), out.stride(0), C.ptr(residual), ldr, ws, wsb, stream)
         C.check(st, "qlin_pro_gemm_i8")
     return out
 
@@ -195,11 +193,10 @@ def pro_proj3(pro: Producer, w1, s1, w2, s2, w3, s3, out, z1=None, z2=None, z3=N
         n1, n2, n3 = ns
         _check_out("out", out, M, n1 + n2 + n3)
         C.require_cuda(*pro.tensors(), w1, s1, w2, s2, w3, s3, z1, z2, z3, out)
-        ws = C.workspace(out.device)
+        ws, wsb, stream = C.scratch(out)
         st = _fn("qlin_pro_proj3_w4")(ctypes.byref(p), M, K, C.ptr(w1), C.ptr(s1), C.ptr(z1), n1, C.ptr(w2),
                                       C.ptr(s2), C.ptr(z2), n2, C.ptr(w3), C.ptr(s3), C.ptr(z3), n3,
-                                      C.dtype_code(s1), grp, C.ptr(out), out.stride(0), C.ptr(ws), ws.numel(),
-                                      C.stream_of(out))
+                                      C.dtype_code(s1), grp, C.ptr(out), out.stride(0), ws, wsb, stream)
         C.check(st, "qlin_pro_proj3_w4")
         return out
     ns = []
@@ -210,10 +207,10 @@ def pro_proj3(pro: Producer, w1, s1, w2, s2, w3, s3, out, z1=None, z2=None, z3=N
     n1, n2, n3 = ns
     _check_out("out", out, M, n1 + n2 + n3)
     C.require_cuda(*pro.tensors(), w1, s1, w2, s2, w3, s3, out)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     st = _fn("qlin_pro_proj3_i8")(ctypes.byref(p), M, K, C.ptr(w1), C.ptr(s1), n1, C.ptr(w2), C.ptr(s2), n2,
                                   C.ptr(w3), C.ptr(s3), n3, C.dtype_code(s1), C.ptr(out), out.stride(0),
-                                  C.ptr(ws), ws.numel(), C.stream_of(out))
+                                  ws, wsb, stream)
     C.check(st, "qlin_pro_proj3_i8")
     return out
 
@@ -233,11 +230,10 @@ def pro_mlp_gate_up_quant(pro: Producer, wg, wsg, wu, wsu, out_q, out_s, zg=None
             raise ValueError("gate and up must have the same N")
         _check_quant_out(out_q, out_s, M, N)
         C.require_cuda(*pro.tensors(), wg, wsg, wu, wsu, zg, zu, out_q, out_s)
-        ws = C.workspace(out_q.device)
+        ws, wsb, stream = C.scratch(out_q)
         st = _fn("qlin_pro_mlp_gate_up_quant_w4")(ctypes.byref(p), M, K, C.ptr(wg), C.ptr(wsg), C.ptr(zg),
                                                   C.ptr(wu), C.ptr(wsu), C.ptr(zu), C.dtype_code(wsg), grp, N,
-                                                  C.ptr(out_q), C.ptr(out_s), C.ptr(ws), ws.numel(),
-                                                  C.stream_of(out_q))
+                                                  C.ptr(out_q), C.ptr(out_s), ws, wsb, stream)
         C.check(st, "qlin_pro_mlp_gate_up_quant_w4")
         return out_q, out_s
     N = _check_w8("wg", wg, wsg, K)
@@ -245,9 +241,9 @@ def pro_mlp_gate_up_quant(pro: Producer, wg, wsg, wu, wsu, out_q, out_s, zg=None
         raise ValueError("gate and up must have the same N")
     _check_quant_out(out_q, out_s, M, N)
     C.require_cuda(*pro.tensors(), wg, wsg, wu, wsu, out_q, out_s)
-    ws = C.workspace(out_q.device)
+    ws, wsb, stream = C.scratch(out_q)
     st = _fn("qlin_pro_mlp_gate_up_quant_i8")(ctypes.byref(p), M, K, C.ptr(wg), C.ptr(wsg), C.ptr(wu),
                                               C.ptr(wsu), C.dtype_code(wsg), N, C.ptr(out_q), C.ptr(out_s),
-                                              C.ptr(ws), ws.numel(), C.stream_of(out_q))
+                                              ws, wsb, stream)
     C.check(st, "qlin_pro_mlp_gate_up_quant_i8")
     return out_q, out_s

@@ -32,7 +32,7 @@ def _check_act(a_q, a_s) -> tuple[int, int]:
     M, K = a_q.shape
     if K % GROUP != 0:
         raise ValueError(f"K={K} must be a multiple of {GROUP}")
-    if a_s.dtype != torch.float32 or tuple(a_s.shape) != (M, K // GROUP):
+    if a_s.dtype != torch.float32 or a_s.shape != (M, K // GROUP):
         raise ValueError(f"a_s must be float32 [M, K/{GROUP}] = [{M}, {K // GROUP}]")
     C.require_contig("a_q", a_q)
     C.require_contig("a_s", a_s)
@@ -75,11 +75,11 @@ def gemm_i8(a_q, a_s, b, b_s, out, residual=None, block_m=None, block_n=None, bl
     if residual is not None:
         _check_out("residual", residual, M, N)
     C.require_cuda(a_q, a_s, b, b_s, out, residual)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_gemm_i8", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(b), C.ptr(b_s), C.dtype_code(b_s), N,
            C.ptr(out), out.stride(0), C.ptr(residual),
            residual.stride(0) if residual is not None else 0,
-           C.ptr(ws), ws.numel(), C.stream_of(out))
+           ws, wsb, stream)
     return out
 
 
@@ -96,9 +96,9 @@ def mlp_gate_up(a_q, a_s, wg, wsg, wu, wsu, out, block_k=64):
     _check_out("out", out, M, N)
     C.require_contig("out", out)
     C.require_cuda(a_q, a_s, wg, wsg, wu, wsu, out)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_mlp_gate_up_i8", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(wg), C.ptr(wsg), C.ptr(wu),
-           C.ptr(wsu), C.dtype_code(wsg), N, C.ptr(out), C.ptr(ws), ws.numel(), C.stream_of(out))
+           C.ptr(wsu), C.dtype_code(wsg), N, C.ptr(out), ws, wsb, stream)
     return out
 
 
@@ -116,19 +116,18 @@ def mlp_gate_up_quant(a_q, a_s, wg, wsg, wu, wsu, out_q, out_s, block_k=64, zg=N
         raise ValueError("gate and up scales must share a dtype")
     _check_quant_out(out_q, out_s, M, N)
     C.require_cuda(a_q, a_s, wg, wsg, wu, wsu, out_q, out_s)
-    ws = C.workspace(out_q.device)
+    ws, wsb, stream = C.scratch(out_q)
     C.call("qlin_mlp_gate_up_quant_i8", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(wg), C.ptr(wsg),
-           C.ptr(wu), C.ptr(wsu), C.dtype_code(wsg), N, C.ptr(out_q), C.ptr(out_s), C.ptr(ws),
-           ws.numel(), C.stream_of(out_q))
+           C.ptr(wu), C.ptr(wsu), C.dtype_code(wsg), N, C.ptr(out_q), C.ptr(out_s), ws, wsb, stream)
     return out_q, out_s
 
 
 def _check_quant_out(out_q, out_s, M, N):
     if N % GROUP != 0:
         raise ValueError(f"N={N} must be a multiple of {GROUP}")
-    if out_q.dtype != torch.int8 or tuple(out_q.shape) != (M, N):
+    if out_q.dtype != torch.int8 or out_q.shape != (M, N):
         raise ValueError(f"out_q must be int8 [{M}, {N}]")
-    if out_s.dtype != torch.float32 or tuple(out_s.shape) != (M, N // GROUP):
+    if out_s.dtype != torch.float32 or out_s.shape != (M, N // GROUP):
         raise ValueError(f"out_s must be float32 [{M}, {N // GROUP}]")
     C.require_contig("out_q", out_q)
     C.require_contig("out_s", out_s)
@@ -150,8 +149,8 @@ def proj3(a_q, a_s, w1, s1, w2, s2, w3, s3, out, block_k=64, z1=None, z2=None, z
     n1, n2, n3 = ns
     _check_out("out", out, M, n1 + n2 + n3)
     C.require_cuda(a_q, a_s, w1, s1, w2, s2, w3, s3, out)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_proj3_i8", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(w1), C.ptr(s1), n1, C.ptr(w2),
            C.ptr(s2), n2, C.ptr(w3), C.ptr(s3), n3, C.dtype_code(s1), C.ptr(out), out.stride(0),
-           C.ptr(ws), ws.numel(), C.stream_of(out))
+           ws, wsb, stream)
     return out

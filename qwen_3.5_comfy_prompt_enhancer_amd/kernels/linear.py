@@ -57,11 +57,10 @@ def linear_w8(x, w, w_scale, out, residual=None):
         if residual.dtype != out.dtype:
             raise ValueError("residual must have the dtype of out")
     C.require_cuda(x, w, w_scale, out, residual)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_linear_w8", C.ptr(x), C.QLIN_F16, M, K, x.stride(0), C.ptr(w), C.ptr(w_scale),
            C.dtype_code(w_scale), N, C.ptr(out), C.dtype_code(out), out.stride(0), C.ptr(residual),
-           residual.stride(0) if residual is not None else 0, C.ptr(ws), ws.numel(),
-           C.stream_of(out))
+           residual.stride(0) if residual is not None else 0, ws, wsb, stream)
     return out
 
 
@@ -77,7 +76,7 @@ def linear_w4(x, w_packed, w_scale, out, w_zero=None, group=None, residual=None)
     if g * w_scale.shape[0] != K or (group is not None and group != g):
         raise ValueError(f"w_scale rows {w_scale.shape[0]} do not match K={K} / group={group}")
     if w_zero is not None:
-        if w_zero.dtype != torch.uint8 or tuple(w_zero.shape) != tuple(w_scale.shape):
+        if w_zero.dtype != torch.uint8 or w_zero.shape != w_scale.shape:
             raise ValueError(f"w_zero must be uint8 {tuple(w_scale.shape)}")
         C.require_contig("w_zero", w_zero)
     C.require_contig("w_packed", w_packed)
@@ -88,12 +87,11 @@ def linear_w4(x, w_packed, w_scale, out, w_zero=None, group=None, residual=None)
         if residual.dtype != out.dtype:
             raise ValueError("residual must have the dtype of out")
     C.require_cuda(x, w_packed, w_scale, w_zero, out, residual)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_linear_w4", C.ptr(x), C.QLIN_F16, M, K, x.stride(0), C.ptr(w_packed),
            C.ptr(w_scale), C.dtype_code(w_scale), C.ptr(w_zero), g, N, C.ptr(out),
            C.dtype_code(out), out.stride(0), C.ptr(residual),
-           residual.stride(0) if residual is not None else 0, C.ptr(ws), ws.numel(),
-           C.stream_of(out))
+           residual.stride(0) if residual is not None else 0, ws, wsb, stream)
     return out
 
 

@@ -214,18 +214,33 @@ def capture(graph: torch.cuda.CUDAGraph, stream: torch.cuda.Stream | None = None
     return torch.cuda.graph(graph, stream=stream, **kw)
 
 
-def require_cuda(*ts) -> torch.device:
-    dev = None
+def scratch(t: torch.Tensor) -> tuple[int, int, int]:
+    """(workspace pointer, its bytes, stream) of a call whose output is `t`: the
+    workspace of t's device and its current stream (see `workspace`)."""
+    idx = t.get_device()
+    if idx < 0:
+        raise ValueError("tensors must be on the GPU")
+    stream = current_stream(idx)
+    w = _ws.get((idx, stream))
+    if w is None:
+        w = workspace(t.device, stream)
+    return w.data_ptr(), w.numel(), stream
+
+
+def require_cuda(*ts) -> None:
+    # device indexes (below 0 off the GPU): torch.device objects took twice as long to
+    # build and compare
+    dev = -2
     for t in ts:
         if t is None:
             continue
-        if not t.is_cuda:
-            raise ValueError("all tensors must be on the GPU")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError("all tensors must be on the same device")
-    return dev
+        idx = t.get_device()
+        if idx != dev:
+            if idx < 0:
+                raise ValueError("all tensors must be on the GPU")
+            if dev >= 0:
+                raise ValueError("all tensors must be on the same device")
+            dev = idx
 
 
 def require_contig(name: str, t) -> None:
@@ -235,10 +250,12 @@ def require_contig(name: str, t) -> None:
 
 def require_rowmajor(name: str, t) -> None:
     """2-D with unit column stride (rows may be strided)."""
-    if t.dim() != 2 or (t.shape[1] > 1 and t.stride(1) != 1):
+    if t.dim() != 2 or (t.stride(1) != 1 and t.shape[1] > 1):
         raise ValueError(f"{name} must be a 2-D row-major matrix")
 
 
 def call(name: str, *args) -> None:
     """Invoke one C entry point and raise on a non-zero status."""
-    check(getattr(lib(), name)(*args), name)
+    status = getattr(_lib or lib(), name)(*args)
+    if status != QLIN_OK:
+        check(status, name)

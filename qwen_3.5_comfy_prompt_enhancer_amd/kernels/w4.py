@@ -31,7 +31,7 @@ def _check_act(a_q, a_s):
     M, K = a_q.shape
     if K % GROUP != 0:
         raise ValueError(f"K={K} must be a multiple of {GROUP}")
-    if a_s.dtype != torch.float32 or tuple(a_s.shape) != (M, K // GROUP):
+    if a_s.dtype != torch.float32 or a_s.shape != (M, K // GROUP):
         raise ValueError(f"a_s must be float32 [M, K/{GROUP}] = [{M}, {K // GROUP}]")
     C.require_contig("a_q", a_q)
     C.require_contig("a_s", a_s)
@@ -51,7 +51,7 @@ def _check_w4(name, w, s, z, K, group=None):
     if group is not None and g != group:
         raise ValueError("all weights of one call must share the weight group")
     if z is not None:
-        if z.dtype != torch.uint8 or tuple(z.shape) != tuple(s.shape):
+        if z.dtype != torch.uint8 or z.shape != s.shape:
             raise ValueError(f"zeros of {name} must be uint8 {tuple(s.shape)}")
         C.require_contig(f"zeros of {name}", z)
     C.require_contig(name, w)
@@ -105,11 +105,10 @@ def gemm_w4(a_q, a_s, b, b_s, out, residual=None, b_z=None, block_m=None, block_
     if residual is not None:
         _check_out("residual", residual, M, N)
     C.require_cuda(a_q, a_s, b, b_s, b_z, out, residual)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_gemm_w4", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(b), C.ptr(b_s), C.dtype_code(b_s),
            C.ptr(b_z), group, N, C.ptr(out), out.stride(0), C.ptr(residual),
-           residual.stride(0) if residual is not None else 0, C.ptr(ws), ws.numel(),
-           C.stream_of(out))
+           residual.stride(0) if residual is not None else 0, ws, wsb, stream)
     return out
 
 
@@ -133,13 +132,12 @@ def proj3_w4(a_q, a_s, w1, s1, w2, s2, w3, s3, out, z1=None, z2=None, z3=None, b
     n1, n2, n3 = ns
     _check_out("out", out, M, n1 + n2 + n3)
     C.require_cuda(a_q, a_s, w1, s1, z1, w2, s2, z2, w3, s3, z3, out)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_proj3_w4", C.ptr(a_q), C.ptr(a_s), M, K,
            C.ptr(w1), C.ptr(s1), C.ptr(z1), n1,
            C.ptr(w2), C.ptr(s2), C.ptr(z2), n2,
            C.ptr(w3), C.ptr(s3), C.ptr(z3), n3,
-           C.dtype_code(s1), group, C.ptr(out), out.stride(0), C.ptr(ws), ws.numel(),
-           C.stream_of(out))
+           C.dtype_code(s1), group, C.ptr(out), out.stride(0), ws, wsb, stream)
     return out
 
 
@@ -162,17 +160,17 @@ def mlp_gate_up_quant_w4(a_q, a_s, wg, sg, wu, su, out_q, out_s, zg=None, zu=Non
     M, K, N, group = _gate_up_common(a_q, a_s, wg, sg, wu, su, zg, zu)
     if N % GROUP != 0:
         raise ValueError(f"N={N} must be a multiple of {GROUP}")
-    if out_q.dtype != torch.int8 or tuple(out_q.shape) != (M, N):
+    if out_q.dtype != torch.int8 or out_q.shape != (M, N):
         raise ValueError(f"out_q must be int8 [{M}, {N}]")
-    if out_s.dtype != torch.float32 or tuple(out_s.shape) != (M, N // GROUP):
+    if out_s.dtype != torch.float32 or out_s.shape != (M, N // GROUP):
         raise ValueError(f"out_s must be float32 [{M}, {N // GROUP}]")
     C.require_contig("out_q", out_q)
     C.require_contig("out_s", out_s)
     C.require_cuda(a_q, a_s, wg, sg, zg, wu, su, zu, out_q, out_s)
-    ws = C.workspace(out_q.device)
+    ws, wsb, stream = C.scratch(out_q)
     C.call("qlin_mlp_gate_up_quant_w4", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(wg), C.ptr(sg),
            C.ptr(zg), C.ptr(wu), C.ptr(su), C.ptr(zu), C.dtype_code(sg), group, N, C.ptr(out_q),
-           C.ptr(out_s), C.ptr(ws), ws.numel(), C.stream_of(out_q))
+           C.ptr(out_s), ws, wsb, stream)
     return out_q, out_s
 
 
@@ -183,12 +181,11 @@ def mlp_gate_up_w4(a_q, a_s, wg, sg, wu, su, out, zg=None, zu=None):
     as mlp_gate_up_quant_w4."""
     zg, zu = fill_zeros((zg, zu), (sg, su), zg if zg is not None else zu)
     M, K, N, group = _gate_up_common(a_q, a_s, wg, sg, wu, su, zg, zu)
-    if out.dtype != torch.bfloat16 or tuple(out.shape) != (M, N):
+    if out.dtype != torch.bfloat16 or out.shape != (M, N):
         raise ValueError(f"out must be bf16 [{M}, {N}]")
     C.require_contig("out", out)
     C.require_cuda(a_q, a_s, wg, sg, zg, wu, su, zu, out)
-    ws = C.workspace(out.device)
+    ws, wsb, stream = C.scratch(out)
     C.call("qlin_mlp_gate_up_w4", C.ptr(a_q), C.ptr(a_s), M, K, C.ptr(wg), C.ptr(sg), C.ptr(zg),
-           C.ptr(wu), C.ptr(su), C.ptr(zu), C.dtype_code(sg), group, N, C.ptr(out), C.ptr(ws),
-           ws.numel(), C.stream_of(out))
+           C.ptr(wu), C.ptr(su), C.ptr(zu), C.dtype_code(sg), group, N, C.ptr(out), ws, wsb, stream)
     return out
