@@ -79,3 +79,38 @@ def test_head_sums_of_every_team_size(hd):
     rq, rs = R.norm_gated_quant_ref(v.float().numpy(), z.float().numpy(), w.float().numpy())
     assert (q.cpu().numpy() == rq).all()
     assert (s.cpu().numpy().view(np.uint32) == rs.astype(np.float32).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("K", [64, 576, 1984, 2048, 2112, 4096, 4160, 6144])
+@pytest.mark.parametrize("dtype,wdt", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_rmsnorm_row_lengths(M, K, dtype, wdt):
+    """Rows of every form: parts of a wave, whole waves, one past them, the long rows."""
+    from qwen35_amd.kernels import norm
+    gen = torch.Generator().manual_seed(K + M)
+    x = torch.randn((M, K + 8), generator=gen).to(dtype)[:, :K]
+    w = torch.randn((K,), generator=gen).to(wdt)
+    q = torch.empty((M, K), dtype=torch.int8, device="cuda")
+    s = torch.empty((M, K // 64), dtype=torch.float32, device="cuda")
+    xg = torch.empty((M, K + 8), dtype=dtype, device="cuda")[:, :K]
+    xg.copy_(x)
+    for one_plus in (True, False):
+        norm.rmsnorm_quant(xg, w.cuda(), q, s, one_plus=one_plus)
+        rq, rs = R.rmsnorm_quant_ref(x.float().numpy(), w.float().numpy(), one_plus=one_plus)
+        assert (q.cpu().numpy() == rq).all()
+        assert (s.cpu().numpy().view(np.uint32) == rs.astype(np.float32).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("N,hd", [(64, 8), (192, 24), (192, 64), (2112, 2112), (4096, 256), (2560, 320)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gate_mul_head_sizes(N, hd, dtype):
+    from qwen35_amd.kernels import norm
+    gen = torch.Generator().manual_seed(N + hd)
+    a = torch.randn((3, N), generator=gen).to(dtype)
+    g = torch.randn((3, 2 * N + 8), generator=gen).to(dtype)
+    q = torch.empty((3, N), dtype=torch.int8, device="cuda")
+    s = torch.empty((3, N // 64), dtype=torch.float32, device="cuda")
+    norm.gate_mul_quant(a.cuda(), g.cuda(), q, s, hd=hd)
+    rq, rs = R.gate_mul_quant_ref(a.float().numpy(), g.float().numpy(), hd)
+    assert (q.cpu().numpy() == rq).all()
+    assert (s.cpu().numpy().view(np.uint32) == rs.astype(np.float32).view(np.uint32)).all()
