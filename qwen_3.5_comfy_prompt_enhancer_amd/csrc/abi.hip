@@ -928,22 +928,29 @@ double plan_kg(int wk, int M, int K, int N, size_t part_cap, long long most, PfP
 
 // Time model of the large tiles (prefill_kernel.h), microseconds: t0 + rounds of 256
 // workgroups (one per CU) x 64-wide K tiles x s + the bytes the tiles read, mb per MB + the
-// split-K exchange, xs per split and xmb per MB of partial tiles; the balanced schedule (256x256
-// only) adds bal and runs sk K tiles.  Fitted to MI355X measurements of every shape and split
-// (M = 150-2048, ten shapes from 1024x3072 to 12288x4096): 2-7 % rms, choices 0.6 % from the
-// best on average.  128x384 is for grids that 256x256 leaves short of or just past a round:
-// W8 2048x6144 M = 1300 46.7 us against 52, 4096x12288 M = 700 85.7 against 92.
+// split-K exchange, xs per split and xmb per MB of partial tiles.  128x128 fits a CU twice: a
+// round of 512 workgroups costs s2 a K tile, one of up to 256 s.  With two K groups a further
+// round costs rr, nothing running beside its start.  The balanced schedule (256x256 only)
+// runs sk K tiles and moves partials of about every tile: 2 + 0.075 a tile.
+// Fitted to MI355X measurements of every shape and split (M = 256-2048, nine shapes from
+// 1024x3072 to 12288x4096), 2-5 % rms; 128x384 carries 3 % more than its fit, since its close
+// calls were lost (W8 2048x6144 at M = 2048 52.5 us against 51.0 on 256x256).  128x128 is for
+// grids of one to two rounds: W8 2048x6144 at M = 1024 36.8 us against 41.5 with two K groups;
+// 128x384 for those 256x256 leaves short of or just past a round: M = 1300 46.7 against 52;
+// the balanced schedule at 4096x12288, M = 2048 184 against 205.
 struct TiledTime {
   int shape;
-  double t0, s, mb, xs, xmb, bal;
+  double t0, s, s2, mb, xs, xmb, rr;
 };
-constexpr TiledTime kTiledTime[2][3] = {  // W8, W4
-    {{PF_256x256, 6.4, 1.240, 0.0203, 1.90, 0.27, 19.9},
-     {PF_128x128_K2, 5.8, 0.438, 0.0105, 0.65, 0.40, -1},
-     {PF_128x384, 6.6, 1.144, 0.0183, -1, 0, -1}},
-    {{PF_256x256, 6.4, 1.548, 0.0183, 1.96, 0.26, 18.3},
-     {PF_128x128_K2, 6.1, 0.590, 0.0078, 0.66, 0.40, -1},
-     {PF_128x384, 6.7, 1.389, 0.0240, -1, 0, -1}}};
+constexpr TiledTime kTiledTime[2][4] = {  // W8, W4
+    {{PF_128x128, 5.39, 0.798, 0.822, 0.0153, 0.900, 0.269, 0},
+     {PF_256x256, 7.34, 1.213, 0, 0.0232, 3.00, 0.127, 0},
+     {PF_128x128_K2, 5.80, 0.438, 0, 0.0105, 0.40, 0.30, 4.5},
+     {PF_128x384, 6.03, 1.201, 0, 0.0294, -1, 0, 0}},
+    {{PF_128x128, 6.07, 0.906, 0.943, 0.0095, 0.737, 0.249, 0},
+     {PF_256x256, 7.15, 1.522, 0, 0.0168, 2.90, 0.133, 0},
+     {PF_128x128_K2, 6.10, 0.590, 0, 0.0078, 0.40, 0.30, 4.0},
+     {PF_128x384, 6.44, 1.445, 0, 0.0264, -1, 0, 0}}};
 
 // The best large-tile plan of a call; *t its time in seconds.
 PfPlan plan_tiled(int wk, int M, int K, int N, size_t part_cap, double* t) {
@@ -953,6 +960,7 @@ PfPlan plan_tiled(int wk, int M, int K, int N, size_t part_cap, double* t) {
   for (const TiledTime& m : kTiledTime[wk == WK_W4]) {
     int bm, bn, waves;
     prefill_geometry(m.shape, &bm, &bn, &waves);
+    const int per_cu = m.s2 > 0 ? 2 : 1;
     const long long tiles = (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     const double base = m.t0 + m.mb * 1e-6 * (double)tiles * K * (2.0 * bm + bn * (wk == WK_W4 ? 0.5 : 1.0));
     const bool counters = tiles <= (long long)(kCounterBytes / sizeof(unsigned));
@@ -962,16 +970,18 @@ PfPlan plan_tiled(int wk, int M, int K, int N, size_t part_cap, double* t) {
     for (int S = 1; S <= 16; S *= 2) {
       const double part = (double)tiles * S * waves * 128 * 64 * sizeof(float);
       if (nk % S != 0 || (S > 1 && (nk / S < 2 || m.xs < 0 || part > (double)part_cap || !counters))) break;
-      if (S > 1 && tiles * (S / 2) >= 256) break;  // split-K exists to fill the chip
-      const double rounds = (double)((tiles * S + 255) / 256);
-      take(base + rounds * (nk / S) * m.s +
+      if (S > 1 && tiles * (S / 2) >= 256LL * per_cu) break;  // split-K exists to fill the chip
+      const long long wgs = tiles * S, rest = wgs % (256 * per_cu);
+      const double rounds = (double)(wgs / (256 * per_cu)) * (per_cu == 2 ? m.s2 : m.s) +
+                            (rest == 0 ? 0.0 : rest > 256 ? m.s2 : m.s);
+      take(base + rounds * (nk / S) + (double)((wgs - 1) / (256 * per_cu)) * m.rr +
                (S > 1 ? m.xs * S + m.xmb * 1e-6 * (double)tiles * S * bm * bn * sizeof(float) : 0.0), S, 0);
     }
     // the balanced schedule: every CU the same run of (tile, K tile) units, across tiles
-    if (m.bal >= 0 && tiles % 256 != 0 && tiles > 128 && counters &&
+    if (m.shape == PF_256x256 && tiles % 256 != 0 && tiles > 128 && counters &&
         (double)tiles * 2 * waves * 128 * 64 * sizeof(float) <= (double)part_cap) {
       const int sk = (int)((tiles * nk + 255) / 256);
-      if (prefill_balanced_ok(tiles, nk, sk)) take(base + m.bal + sk * m.s, 1, sk);
+      if (prefill_balanced_ok(tiles, nk, sk)) take(base + 2.0 + 0.075 * (double)tiles + sk * m.s, 1, sk);
     }
   }
   return best;
