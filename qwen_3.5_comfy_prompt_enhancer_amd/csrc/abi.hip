@@ -936,7 +936,7 @@ double plan_kg(int wk, int M, int K, int N, size_t part_cap, long long most, PfP
 // 1024x3072 to 12288x4096), 2-5 % rms; 128x384 carries 3 % more than its fit, since its close
 // calls were lost (W8 2048x6144 at M = 2048 52.5 us against 51.0 on 256x256).  128x128 is for
 // grids of one to two rounds: W8 2048x6144 at M = 1024 36.8 us against 41.5 with two K groups;
-// 128x384 for those 256x256 leaves short of or just past a round: M = 1300 46.7 against 52;
+// 128x384 for those 256x256 leaves short of a round: W8 2048x6144 M = 1300 46.7 against 52;
 // the balanced schedule at 4096x12288, M = 2048 184 against 205.
 struct TiledTime {
   int shape;
