@@ -107,14 +107,14 @@ void plan_override(const Problem& P, int& cols, int& waves, int& upw) {
 // scale, acc) from zero, in increasing K); split value = lane 0 + lane 1; total =
 // ((v0 + v1) + v2) + ...; then the W8 column scale (and residual, one rounding).
 // The 16-row skinny tiles reproduce it with two waves per split (lanes == 2).
-// S is chosen for the engine's 512-row chunk and a 128-row prompt, then held for every M.
+// S is chosen for the engine's 512-row chunk and then held for every M.
 // Calls with fewer rows (decode: one sequence, or up to eight best-of candidates,
 // engine.py:392) run the engine decode work units (echain.hip), whose results depend
 // on (K, N) and the call kind only, so batch rows equal single rows; a chunk remainder
 // of 1-8 rows therefore agrees with the unchunked prefill to the tolerance, not bit
 // for bit.
 constexpr int kRowsM = kDecodeRowsMax + 1;
-constexpr int kRefChunkM = 512, kRefShortM = 128;
+constexpr int kRefChunkM = 512;
 
 // Column tiles of `tn` over the call's column ranges.
 long long col_tiles(const Problem& P, const SkArgs& a, int tn) {
@@ -211,13 +211,31 @@ int best_tile(const Problem& P, const SkArgs& a, int M, int S, size_t cap, doubl
   return best;
 }
 
-// Split count of the K order: the S (1, 2, 4 or 8, dividing K into ranges of at least
-// two 64-wide blocks) with the least product of the best family's times at the engine's
-// 512-row chunk and at a short prompt of 128 rows.  QLIN_ENGINE_SPLITS overrides it
-// (tuning; it changes the K order).
-int engine_splits(const Problem& call, const SkArgs& a) {
-  Problem P = call;
-  P.hz = false;  // zeros of 8 give the bits of no zeros: the same order for both
+// Microseconds that split_estimate gives the engine's 512-row chunk with S K splits, on
+// 128x128 tiles or on 16-row tiles, whichever is less.  These estimates define the K order
+// (S, and so the bits, of every call of kRowsM rows or more): they stay as they are when the
+// kernels and the time models below change.
+double split_estimate(const Problem& P, const SkArgs& a, int S) {
+  const bool w4 = P.wk == WK_W4;
+  const double elems = (double)P.K * P.ncols * P.nsets / 1e6;
+  const double rows = 5.0 + (w4 ? 0.17 : 0.125) * ((kRefChunkM + 15) / 16) * elems + (S > 1 ? 1.45 * S : 0.0);
+  SkArgs probe = a;
+  probe.M = kRefChunkM;
+  if (!prefill_i8_ok(probe, P.wk, P.epi, I8_128x128)) return rows;
+  const long long wgs = (long long)((kRefChunkM + 127) / 128) * col_tiles(P, a, 128) * S;
+  const double occ = (double)std::min<long long>(wgs, 256);
+  const double stage = (w4 ? 1.8 + 1.6e-3 * occ : 1.05 + 2.5e-3 * occ) * P.nsets;
+  double t = 7.0 + (double)((wgs + 255) / 256) * ((P.K / 64 / S + 1) / 2) * stage;
+  if (S > 1) t += 1.45 * S + 12e-3 * wgs + 0.1e-6 * (double)wgs * P.nsets * 128 * 128 * sizeof(float);
+  return std::min(t, rows);
+}
+
+// Split count of the K order: the S (1, 2, 4 or 8, dividing K into ranges of at least two
+// 64-wide blocks) with the least estimate.  S picked for 128 rows as well as 512, by the tiles'
+// own models, gained at some row counts and lost at others (gemm_i8 12288x4096 at 512 rows
+// 69 -> 81 us, at 2048 243 -> 298; W8 gate/up 4096x12288 at 9 rows 37 -> 61).
+// QLIN_ENGINE_SPLITS overrides it (tuning; it changes the K order).
+int engine_splits(const Problem& P, const SkArgs& a) {
   const int nb = P.K / 64;
   const char* es = getenv("QLIN_ENGINE_SPLITS");
   if (es && *es) return atoi(es);
@@ -227,12 +245,7 @@ int engine_splits(const Problem& call, const SkArgs& a) {
   b.x = nullptr;  // the choice must not depend on where the activations sit
   for (int s = 1; s <= 8; s *= 2) {
     if (nb % s != 0 || (s > 1 && nb / s < 2)) break;
-    double t = 1.0;
-    for (const int m : {kRefChunkM, kRefShortM}) {
-      double tt = 0.0;
-      const double tr = rows_time(P, b, m, s);
-      t *= best_tile(P, b, m, s, kWorkspaceBytes, &tt) >= 0 && tt < tr ? tt : tr;
-    }
+    const double t = split_estimate(P, b, s);
     if (s == 1 || t < best) best = t, S = s;
   }
   return S;

@@ -1,0 +1,39 @@
+"""Which kernels a call launches (csrc/abi.hip, csrc/echain.hip), on the CPU: the library's
+host side over a HIP runtime that records launches."""
+from __future__ import annotations
+
+import pytest
+
+import dispatch as D
+
+
+def _grid(result):
+    st, events, msg = result
+    assert st == 0, msg
+    (launch,) = [e for e in events if e[0] == "launch"]
+    return launch
+
+
+# The K splits of engine calls of nine rows and more are part of their results' definition
+# (the order of fp32 sums): these must not move when kernels or time models change.
+K_SPLITS = [
+    ("i8", 2048, 2048, 1), ("i8", 2048, 6144, 1), ("i8", 6144, 2048, 4), ("i8", 4096, 4096, 2),
+    ("i8", 4096, 12288, 2), ("i8", 12288, 4096, 2), ("i8", 2048, 512, 1), ("i8", 8192, 1024, 8),
+    ("w4", 2048, 2048, 4), ("w4", 4096, 4096, 2), ("w4", 12288, 4096, 2), ("w4", 2048, 512, 1),
+    ("gu8", 2048, 6144, 1), ("gu8", 4096, 12288, 2), ("gu8", 2048, 2048, 4), ("gu8", 1024, 3072, 2),
+    ("gu4", 2048, 6144, 1), ("gu4", 4096, 12288, 2), ("gu4", 512, 256, 1),
+]
+
+
+def test_k_splits(tmp_path):
+    make = {"i8": D.gemm_i8, "w4": D.gemm_w4, "gu8": D.gate_up_i8, "gu4": D.gate_up_w4}
+    # nine rows run on the 16-row tiles: 64 columns without a split, 128 columns x S with
+    got = [_grid(r)[2] for r in D.run(tmp_path, [make[k](9, K, N) for k, K, N, _ in K_SPLITS])]
+    assert got == [N // 64 if s == 1 else -(-N // 128) * s for _, _, N, s in K_SPLITS]
+
+
+def test_calls_without_a_split_need_no_workspace(tmp_path):
+    for st, events, msg in D.run(tmp_path, [f(M, K, N, ws=0) for M in (9, 64, 512) for f, K, N in
+                                            ((D.gemm_i8, 2048, 512), (D.gemm_i8, 2048, 2048), (D.gate_up_w4, 512, 256),
+                                             (D.gate_up_w4, 2048, 6144))]):
+        assert st == 0 and events, msg
