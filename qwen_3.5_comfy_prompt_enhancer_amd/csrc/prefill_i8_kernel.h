@@ -26,16 +26,18 @@
 //     an inline zero, with the weights as its A operand and the activations as B: lane
 //     (g, j) supplies K bytes 16g..16g+15 of weight column 4j + t and of activation row j,
 //     and accumulates 16 adjacent columns of row j.  So it folds one activation scale per
-//     16-row block (four with the operands the other way round: three more registers and
-//     LDS words per block; M = 512, 2048x8192 W8 27.9 -> 26.1 us, gate/up 2048x6144 51.3 ->
-//     46.8, W4 4096x16384 99.9 -> 95.0).  Weight bytes are N-contiguous in
+//     16-row block (four with the operands the other way round: gemm_i8 8192x2048 at M = 512
+//     without a split 72.3 us against 69.3, 2048x6144 25.6 against 24.5; W4 1 %, gate/up
+//     equal).  Weight bytes are N-contiguous in
 //     LDS (as in HBM, rows padded per lane group); each lane reads 4 adjacent columns
 //     of its 16 K rows (one dword per row) and 4x4 byte transposes turn them into the
 //     4 operands.  W4: the nibbles become int8 16 * (n - 8) (even K then odd K), the
 //     activation operand is permuted to the same order, and the scale product carries the
 //     1/16 (exact); explicit zeros add (8 - z) * sum(a) from one more MFMA against all-ones.
-//   * Copies: global -> registers (three stages ahead, two for gate/up) -> LDS (one
-//     stage ahead), one barrier per stage.
+//   * Copies: global -> registers (three stages ahead; two for gate/up and for 160 rows,
+//     whose accumulators leave no second set of registers) -> LDS (one stage ahead), one
+//     barrier per stage.  Every address in the loop is a per-thread value made before it plus
+//     the stage's scalar offset.
 //   * Bound: the fold, two VALU instructions per output and block (three for W4), at about
 //     two thirds of their issue rate.  Reading the next stage's operands into registers
 //     while the current one is folded (three LDS stages) changed nothing (27.9 us at
@@ -171,8 +173,8 @@ void prefill_i8_kernel(const SkArgs a) {
     uint32_t bs;  // W4: raw dword of one group scale of set tid / 256
     uint32_t bz;  // W4 with zeros: the matching zero
   };
-  // The block of every load below is uniform over a wave (its K group k2 is a function of
-  // the wave), so each address is a per-thread offset fixed for the whole loop plus the
+  // The block of every activation and weight load below is uniform over a wave (its K group
+  // is a function of the wave), so each address is a per-thread offset fixed for the whole loop plus the
   // block's offset in a scalar register: buffer loads over the activations, weights and
   // activation scales (the host keeps each under 2^31 bytes), no per-stage address
   // arithmetic on the vector ALU.
@@ -181,34 +183,42 @@ void prefill_i8_kernel(const SkArgs a) {
   __amdgpu_buffer_rsrc_t wr[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) wr[s] = part_rsrc(wset[s], (unsigned)((long long)(W4 ? K / 2 : K) * n));
-  // activation chunk q of a stage: block q / (4 BM), row, 16-byte chunk
-  auto a_chunk = [&](int i, int& k2, int& r, int& c) {
+  // Activation chunk q of a stage: block q / (4 BM), row, 16-byte chunk.  Its block (uniform
+  // over a wave: 4 BM is a multiple of 64), global offset and place in a stage's LDS are
+  // computed once: in the loop, the block's v_readfirstlane kept the compiler from moving any
+  // of it out (382 VALU instructions in two stages instead of 336: gemm_i8 8192x2048 at
+  // M = 1024 without a split 75.0 us against 69.2, gate/up 2048x6144 86.3 against 80.0).
+  constexpr bool XB = THREADS == 4 * BM;  // chunk i is block i's: one offset for both
+  int xk2[NA];
+  unsigned xoff[NA], xdst[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
     const int q = tid + THREADS * i;
-    k2 = (int)rfl((uint32_t)(q / (4 * BM)));  // uniform over a wave: 4 BM is a multiple of 64
-    r = (q - 4 * BM * k2) >> 2;
-    c = q & 3;
-  };
+    xk2[i] = XB ? i : (int)rfl((uint32_t)(q / (4 * BM)));
+    const int r = (XB ? tid : q - 4 * BM * xk2[i]) >> 2, c = tid & 3;
+    xoff[i] = (unsigned)(min(m0 + r, M - 1) * K + 16 * c);
+    xdst[i] = (unsigned)(xk2[i] * G::A_BLK + a_off(r, c));
+  }
   constexpr int BCH = BN / 16;                    // 16-byte chunks of a weight row
   constexpr int BPB = (W4 ? 32 : 64) * BCH;       // and of a block
   const int wk2 = W4 ? (int)rfl((uint32_t)tid / BPB) : 0;
   const int wrow = (tid % BPB) / BCH, wch = tid % BCH;  // W8: block i's row and chunk alike
-  unsigned xoff[NA];
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    int k2, r, c;
-    a_chunk(i, k2, r, c);
-    xoff[i] = (unsigned)(min(m0 + r, M - 1) * K + 16 * c);
-  }
   const unsigned woff = (unsigned)(wrow * n + ncol0 + 16 * wch);
+  const unsigned wdst = (unsigned)(wk2 * G::B_BLK + G::b_row(wrow) + 16 * wch);
+  // activation scale e of a stage: block e / BM, row e % BM
+  constexpr bool SU = BM % 64 == 0;  // its block is uniform over a wave
+  int sk2[NAS];
   unsigned soff[NAS];
 #pragma unroll
-  for (int i = 0; i < NAS; ++i) soff[i] = (unsigned)(min(m0 + (tid + THREADS * i) % BM, M - 1) * NG * 4);
+  for (int i = 0; i < NAS; ++i) {
+    const int e = tid + THREADS * i;
+    sk2[i] = SU ? (int)rfl((uint32_t)(e / BM)) : e / BM;
+    soff[i] = (unsigned)(min(m0 + e % BM, M - 1) * NG * 4);
+  }
   auto fetch = [&](Regs& rg, int st) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      int k2, r, c;
-      a_chunk(i, k2, r, c);
-      const int blk = kb0 + min(2 * st + k2, nk - 1);
+      const int blk = kb0 + min(2 * st + xk2[i], nk - 1);
       rg.av[i] = bitcast<u32x4>(__builtin_amdgcn_raw_buffer_load_b128(xr, xoff[i], blk * 64, 0));
     }
 #pragma unroll
@@ -228,8 +238,9 @@ void prefill_i8_kernel(const SkArgs a) {
     for (int i = 0; i < NAS; ++i) {
       const int e = tid + THREADS * i;
       if (e < 2 * BM) {
-        const int blk = kb0 + min(2 * st + e / BM, nk - 1);
-        rg.as_[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff[i] + 4 * blk, 0, 0));
+        const int blk = kb0 + min(2 * st + sk2[i], nk - 1);
+        rg.as_[i] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff[i] + (SU ? 0 : 4 * blk), SU ? 4 * blk : 0, 0));
       }
     }
     if constexpr (W4) {
@@ -248,19 +259,15 @@ void prefill_i8_kernel(const SkArgs a) {
   auto store = [&](const Regs& rg, int buf) {
     uint8_t* base = lds + buf * G::STAGE;
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      int k2, r, c;
-      a_chunk(i, k2, r, c);
-      *(u32x4*)(base + k2 * G::A_BLK + a_off(r, c)) = rg.av[i];
-    }
+    for (int i = 0; i < NA; ++i) *(u32x4*)(base + xdst[i]) = rg.av[i];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       uint8_t* sb = base + G::B_OFF + s * 2 * G::B_BLK;
       if constexpr (W4) {
-        *(u32x4*)(sb + wk2 * G::B_BLK + G::b_row(wrow) + 16 * wch) = rg.bv[s][0];
+        *(u32x4*)(sb + wdst) = rg.bv[s][0];
       } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) *(u32x4*)(sb + i * G::B_BLK + G::b_row(wrow) + 16 * wch) = rg.bv[s][i];
+        for (int i = 0; i < 2; ++i) *(u32x4*)(sb + i * G::B_BLK + wdst) = rg.bv[s][i];
       }
     }
 #pragma unroll
@@ -301,19 +308,22 @@ void prefill_i8_kernel(const SkArgs a) {
     i32x4 av[RB];
     float as[RB];
   };
+  // (one address per operand and compile-time steps from it: 16 rows on, a row's chunks are
+  // swizzled alike.  With the addresses above, 20-70 registers fewer.)
+  const unsigned asrc = (unsigned)(kg * G::A_BLK + a_off(wm * 16 * RB + j, g));
+  const unsigned ssrc = (unsigned)(G::AS_OFF + (kg * BM + wm * 16 * RB + j) * 4);
+  const unsigned wsrc = (unsigned)(G::B_OFF + kg * G::B_BLK + G::b_row(G::RG * g) + cb);
+  const unsigned bsrc = (unsigned)((kg * BN + ccol) * 4);
   auto load_a = [&](const uint8_t* base, Aop& o) {
-    const uint8_t* sa = base + kg * G::A_BLK;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      const int r = wm * 16 * RB + rb * 16 + j;
-      o.av[rb] = *(const i32x4*)(sa + a_off(r, g));
-      o.as[rb] = *(const float*)(base + G::AS_OFF + (kg * BM + r) * 4);
+      o.av[rb] = *(const i32x4*)(base + asrc + rb * 1024);
+      o.as[rb] = *(const float*)(base + ssrc + rb * 64);
     }
   };
   auto load_w = [&](const uint8_t* base, int s, Wop& o) {
-    const uint8_t* sb = base + G::B_OFF + (s * 2 + kg) * G::B_BLK;
 #pragma unroll
-    for (int i = 0; i < (W4 ? 8 : 16); ++i) o.d[i] = *(const uint32_t*)(sb + G::b_row((W4 ? 8 : 16) * g + i) + cb);
+    for (int i = 0; i < G::RG; ++i) o.d[i] = *(const uint32_t*)(base + wsrc + s * 2 * G::B_BLK + i * BN);
   };
   // columns whose dots are computed before their folds (4 RB registers each), so that the
   // folds run back to back instead of each waiting on its MFMA
@@ -326,8 +336,8 @@ void prefill_i8_kernel(const SkArgs a) {
     if constexpr (W4) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        bs[r] = *(const f32x4*)(base + G::BS_OFF + ((s * 2 + kg) * BN + ccol + 4 * r) * 4);
-        if constexpr (HZ) zc[r] = *(const i32x4*)(base + G::BZ_OFF + ((s * 2 + kg) * BN + ccol + 4 * r) * 4);
+        bs[r] = *(const f32x4*)(base + G::BS_OFF + bsrc + (s * 2 * BN + 4 * r) * 4);
+        if constexpr (HZ) zc[r] = *(const i32x4*)(base + G::BZ_OFF + bsrc + (s * 2 * BN + 4 * r) * 4);
       }
     }
     u32x4 bv[4];
