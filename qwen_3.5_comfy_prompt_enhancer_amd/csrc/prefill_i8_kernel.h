@@ -292,33 +292,51 @@ void prefill_i8_kernel(const SkArgs a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc[s][rb][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const i32x4 izero = i32x4{0, 0, 0, 0};
-  // The weights are the MFMA's A operand and the activations its B operand: lane (g, j)
+  // WA: the weights are the MFMA's A operand and the activations its B operand: lane (g, j)
   // holds, of instruction t, D rows 4g + r = weight columns 16g + 4r + t and D column j =
   // activation row j.  So a lane folds one activation row per block of 16 (one a_s value
-  // instead of four) and ends with 16 adjacent columns of it.
-  const int cb = wn * 64 + 4 * j;    // first of the 4 columns whose operand the lane builds
-  const int ccol = wn * 64 + 16 * g;  // first of the 16 columns the lane accumulates
+  // instead of four) and ends with 16 adjacent columns of it.  With zeros the other way
+  // round: lane (g, j) ends with columns 4j .. 4j + 3 of rows 4g + r, and holds 4 group
+  // scales and 4 zeros instead of 16 of each, which gate/up's registers have no room for
+  // (its loop reloaded spilled addresses, waiting for the copies in flight: 4096x12288 at
+  // M = 512 on 128x128 276 us against 210; store calls within 3 % but for 160 rows, 6 % behind).
+  constexpr bool WA = !HZ;
+  auto mfma = [](i32x4 w, i32x4 x) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(WA ? w : x, WA ? x : w, i32x4{0, 0, 0, 0}, 0, 0, 0);
+  };
+  constexpr int LC = WA ? 16 : 4, LR = 16 / LC;  // columns and rows (per block of 16) of a lane
+  const int cb = wn * 64 + 4 * j;                // first of the 4 columns whose operand the lane builds
+  const int ccol = WA ? wn * 64 + 16 * g : cb;   // first of the columns the lane accumulates
+  using ScaleA = std::conditional_t<WA, float, f32x4>;  // a lane's activation scales of a block of 16 rows
 
-  // Operands of one 64-wide block of one weight set, raw from LDS.
+  // Operands of one 64-wide block: a weight set's raw from LDS, and the activations'.
   struct Wop {
     uint32_t d[W4 ? 8 : 16];
   };
   struct Aop {
     i32x4 av[RB];
-    float as[RB];
+    ScaleA as[RB];
+    i32x4 sx[HZ ? RB : 1];  // W4 with zeros: sums of the rows' codes (every column alike)
   };
   // (one address per operand and compile-time steps from it: 16 rows on, a row's chunks are
-  // swizzled alike.  With the addresses above, 20-70 registers fewer.)
+  // swizzled alike)
   const unsigned asrc = (unsigned)(kg * G::A_BLK + a_off(wm * 16 * RB + j, g));
-  const unsigned ssrc = (unsigned)(G::AS_OFF + (kg * BM + wm * 16 * RB + j) * 4);
+  const unsigned ssrc = (unsigned)(G::AS_OFF + (kg * BM + wm * 16 * RB + (WA ? j : 4 * g)) * 4);
   const unsigned wsrc = (unsigned)(G::B_OFF + kg * G::B_BLK + G::b_row(G::RG * g) + cb);
   const unsigned bsrc = (unsigned)((kg * BN + ccol) * 4);
   auto load_a = [&](const uint8_t* base, Aop& o) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       o.av[rb] = *(const i32x4*)(base + asrc + rb * 1024);
-      o.as[rb] = *(const float*)(base + ssrc + rb * 64);
+      o.as[rb] = *(const ScaleA*)(base + ssrc + rb * 64);
+      if constexpr (W4) {
+        // slots in the order of the nibble split: even K of the 16, then odd K
+        const u32x4 x = bitcast<u32x4>(o.av[rb]);
+        o.av[rb] = bitcast<i32x4>(u32x4{perm(x.y, x.x, 0x06040200u), perm(x.w, x.z, 0x06040200u),
+                                        perm(x.y, x.x, 0x07050301u), perm(x.w, x.z, 0x07050301u)});
+      }
+      if constexpr (HZ)
+        o.sx[rb] = mfma(bitcast<i32x4>(u32x4{0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u}), o.av[rb]);
     }
   };
   auto load_w = [&](const uint8_t* base, int s, Wop& o) {
@@ -331,31 +349,17 @@ void prefill_i8_kernel(const SkArgs a) {
   // folds one block of set s; W4 group scales and zeros come from the stage (`base`) here,
   // where they are used, and take no registers before
   auto fold = [&](int s, const uint8_t* base, const Aop& A, const Wop& B) {
-    f32x4 bs[4];
-    i32x4 zc[4];
+    f32x4 bs[LC / 4];
+    i32x4 zc[LC / 4];
     if constexpr (W4) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      for (int r = 0; r < LC / 4; ++r) {
         bs[r] = *(const f32x4*)(base + G::BS_OFF + bsrc + (s * 2 * BN + 4 * r) * 4);
         if constexpr (HZ) zc[r] = *(const i32x4*)(base + G::BZ_OFF + bsrc + (s * 2 * BN + 4 * r) * 4);
       }
     }
     u32x4 bv[4];
-    i32x4 av[RB];
-    i32x4 sx[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) av[rb] = A.av[rb];
     if constexpr (W4) {
-      // activation slots in the order of the nibble split: even K of the 16, then odd K
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const u32x4 x = bitcast<u32x4>(A.av[rb]);
-        av[rb] = bitcast<i32x4>(u32x4{perm(x.y, x.x, 0x06040200u), perm(x.w, x.z, 0x06040200u),
-                                      perm(x.y, x.x, 0x07050301u), perm(x.w, x.z, 0x07050301u)});
-        if constexpr (HZ)  // sum of the row's codes (every D row alike)
-          sx[rb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-              bitcast<i32x4>(u32x4{0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u}), av[rb], izero, 0, 0, 0);
-      }
       uint32_t lo[8], hi[8], e0[4], e1[4], o0[4], o1[4];
 #pragma unroll
       for (int i = 0; i < 8; ++i) w4_split_i8x16(B.d[i], lo[i], hi[i]);
@@ -381,7 +385,7 @@ void prefill_i8_kernel(const SkArgs a) {
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int t = 0; t < DOTS; ++t)
-          p[rb][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bitcast<i32x4>(bv[t0 + t]), av[rb], izero, 0, 0, 0);
+          p[rb][t] = mfma(bitcast<i32x4>(bv[t0 + t]), A.av[rb]);
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -389,16 +393,19 @@ void prefill_i8_kernel(const SkArgs a) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float c = acc[s][rb][t0 + t][r];
+            float as;
+            if constexpr (WA) as = A.as[rb];
+            else as = A.as[rb][r];
             if constexpr (W4) {
               // The MFMA sums 16 * (nibble - 8) * a: the dot is p / 16, exactly.  Rather
               // than shifting every p, the fold takes float(p) (exact: |p| < 2^24) against
               // the scale product divided by 16 (exact): fma(float(p), fl(a_s * b_s) / 16,
               // acc) is fma(float(p / 16), fl(a_s * b_s), acc) bit for bit.
               int v = p[rb][t][r];
-              if constexpr (HZ) v += zc[r][t0 + t] * sx[rb][0];
-              acc[s][rb][t0 + t][r] = fmaf((float)v, A.as[rb] * bs[r][t0 + t], c);
+              if constexpr (HZ) v += zc[WA ? r : 0][t0 + t] * A.sx[rb][WA ? 0 : r];
+              acc[s][rb][t0 + t][r] = fmaf((float)v, as * bs[WA ? r : 0][t0 + t], c);
             } else {
-              acc[s][rb][t0 + t][r] = fmaf((float)p[rb][t][r], A.as[rb], c);
+              acc[s][rb][t0 + t][r] = fmaf((float)p[rb][t][r], as, c);
             }
           }
     }
@@ -466,11 +473,11 @@ void prefill_i8_kernel(const SkArgs a) {
     }
   }
   // W8 column scales of the epilogue: in flight during the sums below
-  u32x4 csraw[NS][4];
+  u32x4 csraw[NS][LC / 4];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < LC / 4; ++r)
       csraw[s][r] = W4 ? u32x4{0u, 0u, 0u, 0u} : ld_scale4_raw(sset[s], a.sdt, ncol0 + ccol + 4 * r);
 
   // ---------------- K groups: group 0 + group 1 (fixed order), one set at a time ----------------
@@ -555,18 +562,20 @@ void prefill_i8_kernel(const SkArgs a) {
   }
 
   // ---------------- epilogue ----------------
-  // Lane (g, j): columns 16g .. 16g + 15 of the wave's 64 (column 4r + t of them in
-  // acc[..][t][r]) of row j of each block of 16.
-  const int col = ncol0 + ccol;  // within the matrix
-  float cs[NS][16];
+  // Value (i, c) of a lane's block of 16 rows: its row i (of LR) and column c (of LC).
+  const int col = ncol0 + ccol;  // its first column within the matrix
+  auto val = [&](int s, int rb, int i, int c) { return WA ? acc[s][rb][c & 3][c >> 2] : acc[s][rb][c & 3][i]; };
+  float cs[NS][LC];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < LC / 4; ++r) {
       if constexpr (W4) cs[s][4 * r] = cs[s][4 * r + 1] = cs[s][4 * r + 2] = cs[s][4 * r + 3] = 1.0f;
       else cvt_scale4(csraw[s][r], a.sdt, &cs[s][4 * r]);
     }
-  const int r0 = m0 + wm * 16 * RB + j;
+  const int r0 = m0 + wm * 16 * RB + (WA ? j : 4 * g);
+  constexpr int VC = LC < 8 ? LC : 8;  // 16-bit values of a store
+  using V16 = std::conditional_t<VC == 8, u32x4, u32x2>;
   if constexpr (EPI == EPI_STORE) {
     // column scale (W8), residual, 16-bit store.  The output type and the residual
     // are uniform: branch once, outside the per-value code.
@@ -578,30 +587,34 @@ void prefill_i8_kernel(const SkArgs a) {
         else return bitcast<uint32_t>(__builtin_convertvector((float __attribute__((ext_vector_type(2)))){v0, v1}, f16x2));
       };
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int row = r0 + rb * 16;
-        if (!mine(rb) || row >= M) continue;
-        uint16_t* const o = (uint16_t*)a.out + (long long)row * a.ldo + ocol;
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          // column scale and residual in one rounding (fmaf), the product alone
-          // without a residual: the skinny kernel's epilogue rounds the same way
-          u32x4 rv = u32x4{0u, 0u, 0u, 0u};
-          if constexpr (RES) rv = *(const u32x4*)((const uint16_t*)a.res + (long long)row * a.ldr + ocol + 8 * h);
-          float y[8];
+        for (int i = 0; i < LR; ++i) {
+          const int row = r0 + rb * 16 + i;
+          if (!mine(rb) || row >= M) continue;
+          uint16_t* const o = (uint16_t*)a.out + (long long)row * a.ldo + ocol;
 #pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            const float v = acc[0][rb][c & 3][2 * h + (c >> 2)], k = cs[0][8 * h + c];
-            if constexpr (RES) {
-              const uint16_t hh = (uint16_t)(rv[c >> 1] >> (16 * (c & 1)));
-              y[c] = fmaf(v, k, BF ? bf16_to_f32(hh) : (float)bitcast<_Float16>(hh));
-            } else {
-              y[c] = v * k;
+          for (int h = 0; h < LC / VC; ++h) {
+            // column scale and residual in one rounding (fmaf), the product alone
+            // without a residual: the skinny kernel's epilogue rounds the same way
+            V16 rv = V16(0u), ov;
+            if constexpr (RES) rv = *(const V16*)((const uint16_t*)a.res + (long long)row * a.ldr + ocol + VC * h);
+            float y[VC];
+#pragma unroll
+            for (int c = 0; c < VC; ++c) {
+              const float v = val(0, rb, i, VC * h + c), k = cs[0][VC * h + c];
+              if constexpr (RES) {
+                const uint16_t hh = (uint16_t)(rv[c >> 1] >> (16 * (c & 1)));
+                y[c] = fmaf(v, k, BF ? bf16_to_f32(hh) : (float)bitcast<_Float16>(hh));
+              } else {
+                y[c] = v * k;
+              }
             }
+#pragma unroll
+            for (int c = 0; c < VC / 2; ++c) ov[c] = cvt2(y[2 * c], y[2 * c + 1]);
+            *(V16*)(o + VC * h) = ov;
           }
-          *(u32x4*)(o + 8 * h) = u32x4{cvt2(y[0], y[1]), cvt2(y[2], y[3]), cvt2(y[4], y[5]), cvt2(y[6], y[7])};
         }
-      }
     };
     using T = std::true_type;
     using F = std::false_type;
@@ -614,48 +627,62 @@ void prefill_i8_kernel(const SkArgs a) {
     }
   } else {
     // h = silu(g) * u; bf16 store, or bf16 round trip and per-64-column int8 quant.
-    // A row's 64 columns of this wave tile are the four lanes g of its j (16 columns
-    // each): the amax reduces over those lanes.
+    // A row's 64 columns of this wave tile are the four lanes g of its j (WA) or the
+    // sixteen lanes j of its g: the amax reduces over those lanes.
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       if (!mine(rb)) continue;
-      const int row = r0 + rb * 16;
-      float h[16];
 #pragma unroll
-      for (int c = 0; c < 16; ++c)
-        h[c] = silu(acc[0][rb][c & 3][c >> 2] * cs[0][c]) * (acc[1][rb][c & 3][c >> 2] * cs[1][c]);
-      if constexpr (EPI == EPI_GATEUP) {
-        if (row < M) {
-          uint32_t o[8];
+      for (int i = 0; i < LR; ++i) {
+        const int row = r0 + rb * 16 + i;
+        float h[LC];
 #pragma unroll
-          for (int c = 0; c < 8; ++c)
-            o[c] = (uint32_t)f32_to_bf16(h[2 * c]) | ((uint32_t)f32_to_bf16(h[2 * c + 1]) << 16);
-          uint16_t* const d = (uint16_t*)a.out + (long long)row * a.ncols + col;
-          *(u32x4*)d = u32x4{o[0], o[1], o[2], o[3]};
-          *(u32x4*)(d + 8) = u32x4{o[4], o[5], o[6], o[7]};
-        }
-      } else {
-        float am = 0.0f;
+        for (int c = 0; c < LC; ++c) h[c] = silu(val(0, rb, i, c) * cs[0][c]) * (val(1, rb, i, c) * cs[1][c]);
+        if constexpr (EPI == EPI_GATEUP) {
+          if (row < M) {
+            uint16_t* const d = (uint16_t*)a.out + (long long)row * a.ncols + col;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          h[c] = bf16_to_f32(f32_to_bf16(h[c]));  // bf16 round trip (kernels/gemm.py:198-200)
-          am = fmaxf(am, fabsf(h[c]));
-        }
-        float am0, am1;
-        lane_pair<16>(am, am0, am1);
-        lane_pair<32>(fmaxf(am0, am1), am0, am1);
-        const float sc = fmaxf(fmaxf(am0, am1) / 127.0f, 1e-8f);
-        const float inv = 1.0f / sc;
-        if (row < M) {
-          uint32_t qw[4];
+            for (int v = 0; v < LC / VC; ++v) {
+              V16 o;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            qw[q] = 0;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) qw[q] |= ((uint32_t)(quant_i8(h[4 * q + t], sc, inv) & 0xFF)) << (8 * t);
+              for (int c = 0; c < VC / 2; ++c)
+                o[c] = (uint32_t)f32_to_bf16(h[VC * v + 2 * c]) | ((uint32_t)f32_to_bf16(h[VC * v + 2 * c + 1]) << 16);
+              *(V16*)(d + VC * v) = o;
+            }
           }
-          *(u32x4*)(a.oq + (long long)row * a.ncols + col) = u32x4{qw[0], qw[1], qw[2], qw[3]};
-          if (g == 0) a.os[(long long)row * (a.ncols / 64) + col / 64] = sc;
+        } else {
+          float am = 0.0f;
+#pragma unroll
+          for (int c = 0; c < LC; ++c) {
+            h[c] = bf16_to_f32(f32_to_bf16(h[c]));  // bf16 round trip (kernels/gemm.py:198-200)
+            am = fmaxf(am, fabsf(h[c]));
+          }
+          if constexpr (WA) {
+            float am0, am1;
+            lane_pair<16>(am, am0, am1);
+            lane_pair<32>(fmaxf(am0, am1), am0, am1);
+            am = fmaxf(am0, am1);
+          } else {
+            am = fmaxf(am, lane_xor<1>(am));
+            am = fmaxf(am, lane_xor<2>(am));
+            am = fmaxf(am, lane_xor<4>(am));
+            am = fmaxf(am, lane_xor<8>(am));
+          }
+          const float sc = fmaxf(am / 127.0f, 1e-8f);
+          const float inv = 1.0f / sc;
+          if (row < M) {
+            uint32_t qw[LC / 4];
+#pragma unroll
+            for (int q = 0; q < LC / 4; ++q) {
+              qw[q] = 0;
+#pragma unroll
+              for (int t = 0; t < 4; ++t) qw[q] |= ((uint32_t)(quant_i8(h[4 * q + t], sc, inv) & 0xFF)) << (8 * t);
+            }
+            int8_t* const d = a.oq + (long long)row * a.ncols + col;
+            if constexpr (WA) *(u32x4*)d = u32x4{qw[0], qw[1], qw[2], qw[3]};
+            else *(uint32_t*)d = qw[0];
+            if (WA ? g == 0 : j == 0) a.os[(long long)row * (a.ncols / 64) + col / 64] = sc;
+          }
         }
       }
     }

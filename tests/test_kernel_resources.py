@@ -59,3 +59,11 @@ def test_small_prefill_tiles_leave_room_for_three_waves():
                  "Li1ELb0ELi0ELi2ELi1E", "Li1ELb0ELi1ELi2ELi1E", "Li1ELb0ELi2ELi2ELi1E"):
         for k in _find("prefill_i8_kernelI" + part):
             assert k[".vgpr_count"] <= 168, k[".name"]
+
+
+def test_prefill_tiles_do_not_spill_in_their_loops():
+    """A spilled register that the K loop reloads makes every stage wait for its copies in
+    flight.  The few that remain (up to three, W4 gate/up with zeros) are stored and read
+    outside it."""
+    for k in _find("prefill_i8_kernel"):
+        assert k[".vgpr_spill_count"] <= 3, (k[".name"], k[".vgpr_spill_count"])
