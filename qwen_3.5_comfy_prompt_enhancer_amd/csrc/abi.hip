@@ -124,45 +124,62 @@ long long col_tiles(const Problem& P, const SkArgs& a, int tn) {
 }
 
 // Time models (microseconds) of the kernel families of an engine call of M rows split S
-// ways, fitted to MI355X measurements of every tile and of the 16-row tiles (M = 17-700,
-// S = 1, 2, 4, W8 and W4-g128, layer shapes 1024x1024 to 4096x16384 and 12288x4096, gate/up
-// 2048x6144 and 4096x12288, weights rotated so that they stream from HBM):
+// ways, for the choice between them (it changes no bits):
 //   tiled: t0 + 128-wide K stages x s[q - 1] for each round of q workgroups per CU (`cap` of
-//          them are resident at once) + the split-K exchange, xs per split and xmb per MB of
-//          partial tiles.  4 % rms from the measurements, 15 % at most.
-//   rows:  t0 + 64-wide block pairs x (c0 + c1 x workgroups per CU) + the exchange.  10 % rms.
+//          them are resident at once) + wmb per MB of weights + the split-K exchange, xs per
+//          split and xmb per MB of partial tiles
+//   rows:  t0 + 64-wide block pairs x (c0 + c1 x workgroups per CU) + the exchange
+// Fitted to MI355X measurements of every tile and of the 16-row tiles at the calls' own splits
+// (M = 17-4096 at 25 row counts, 41 shapes from 2048x64 to 12288x4096 and 3584x18944, one set
+// and gate/up, weights rotated so that they stream from HBM), then moved where that let the
+// choice agree with the measurements: over those 4626 calls the chosen kernel is 0.4 % behind
+// the fastest.  (A fit over one workgroup count per shape, without the weights' term, chose
+// 96x64 tiles for gemm_i8 4096x12288 at 96 rows: 36 us against 28 on 128x128.)
 struct TileTime {
-  double t0, s[3], xs, xmb;
+  double t0, s[3], xs, xmb, wmb;
   int cap;
 };
 struct RowsTime {
   double t0, c0, c1, xs, xw;
 };
-constexpr TileTime kTileTime[2][2][I8_TILES] = {
+constexpr TileTime kTileTime[3][2][I8_TILES] = {
     // W8: 128x128, 64x64, 96x64, 128x64, 160x64; one weight set, then gate/up
-    {{{6.2, {1.10, 0, 0}, 0.81, 0.394, 1},
-      {4.7, {0.67, 0.90, 1.17}, 0.51, 0.349, 3},
-      {5.5, {0.81, 1.14, 0}, 0.43, 0.389, 2},
-      {6.0, {1.02, 1.42, 0}, 0.54, 0.347, 2},
-      {6.4, {1.15, 1.64, 0}, 0.60, 0.303, 2}},
-     {{7.6, {2.22, 0, 0}, 3.1, 0.81, 1}, {8.7, {1.02, 1.54, 0}, 0, 0.48, 2}, {9.8, {1.36, 1.89, 0}, 0, 0.466, 2}}},
+    {{{5.27, {1, 0, 0}, 0.693, 0.477, 0.00798, 1},
+      {4.03, {0.527, 0.755, 1.17}, 0.41, 0.355, 0.0985, 3},
+      {6.21, {0.604, 0.965, 1.51}, 0.993, 0.32, 0.0599, 3},
+      {5.27, {0.868, 1.34, 0}, 0.721, 0.351, 0.0278, 2},
+      {5.32, {1.05, 1.69, 0}, 1.49, 0.272, 0.0402, 2}},
+     {{8.42, {1.99, 0, 0}, 0.952, 0.407, 0.00836, 1},
+      {9.78, {0.791, 1.2, 1.91}, 0.556, 0.281, 0.0284, 3},
+      {8.62, {1.04, 1.72, 0}, 1.51, 0.362, 0.0899, 2}}},
     // W4
-    {{{5.5, {1.32, 0, 0}, 0.75, 0.375, 1},
-      {5.3, {0.81, 1.11, 1.34}, 0.40, 0.273, 3},
-      {5.7, {1.06, 1.35, 0}, 0.35, 0.372, 2},
-      {6.0, {1.26, 1.60, 0}, 0.44, 0.339, 2},
-      {6.5, {1.53, 2.02, 0}, 0.49, 0.285, 2}},
-     {{8.2, {2.75, 0, 0}, 0.58, 0.459, 1}, {8.5, {1.33, 1.77, 0}, 0, 0.45, 2}, {9.6, {1.70, 2.21, 0}, 0, 0.427, 2}}}};
-constexpr RowsTime kRowsTime[2][2][2] = {  // [W8, W4][one set, gate/up][S = 1, S > 1]
-    {{{4.0, 0.143, 0.264, 0, 0}, {8.1, 0, 0.739, 0.31, 1.085}},
-     {{6.0, 0.648, 0.369, 0, 0}, {12.1, 0.098, 1.589, 0, 2.04}}},
-    {{{5.5, 0.272, 0.208, 0, 0}, {8.6, 0.509, 0.255, 0, 1.91}},
-     {{7.9, 0.471, 0.368, 0, 0}, {5.8, 0.866, 0.688, 0, 6.62}}}};
-// explicit zeros cost an instruction per output and block (measured 1.2-1.3 x per stage)
-constexpr double kZerosFactor = 1.25;
+    {{{3.61, {1.27, 0, 0}, 0.539, 0.423, 0.05, 1},
+      {4.38, {0.605, 0.992, 1.23}, 0.67, 0.24, 0.0716, 3},
+      {4.77, {0.888, 1.18, 0}, 1.05, 0.384, 0.0926, 2},
+      {5.14, {1.08, 1.5, 0}, 0.816, 0.305, 0.047, 2},
+      {5.46, {1.39, 2.01, 0}, 1.49, 0.229, 0.00759, 2}},
+     {{7.67, {2.53, 0, 0}, 0.833, 0.392, 0, 1},
+      {6.41, {0.778, 1.53, 2.06}, 0.965, 0.277, 0.0689, 3},
+      {7.89, {1.43, 1.94, 0}, 1.75, 0.352, 0.078, 2}}},
+    // W4 with zeros
+    {{{3.87, {1.57, 0, 0}, 0.614, 0.418, 0.0639, 1},
+      {4.88, {0.694, 1.16, 1.45}, 0.617, 0.224, 0.0565, 3},
+      {5.09, {1.12, 1.41, 0}, 0.991, 0.384, 0.0301, 2},
+      {5.99, {1.3, 1.61, 0}, 0.68, 0.392, 0.0575, 2},
+      {6.79, {1.72, 2.23, 0}, 1.47, 0.284, 0.0386, 2}},
+     {{10.6, {2.98, 0, 0}, 1.17, 0.417, 0.00702, 1},
+      {6.71, {1.05, 1.97, 0}, 1.02, 0.336, 0.0333, 2},
+      {7.96, {1.93, 2.34, 0}, 1.75, 0.441, 0.0158, 2}}}};
+constexpr RowsTime kRowsTime[3][2][2] = {  // [W8, W4, W4 with zeros][one set, gate/up][S = 1, S > 1]
+    {{{4.3, 0.114, 0.376, 0, 0}, {9.68, 0.0748, 0.644, 0, 1.25}}, {{4.92, 0.601, 0.479, 0, 0}, {14.6, 0, 1.54, 0, 0.497}}},
+    {{{5, 0.277, 0.184, 0, 0}, {8.86, 0.441, 0.282, 0.0523, 1.84}}, {{6.59, 0.455, 0.285, 0, 0}, {12, 0.454, 0.783, 0.143, 5.72}}},
+    {{{6.07, 0.339, 0.186, 0, 0}, {8.87, 0.525, 0.328, 0.0555, 1.83}}, {{6.14, 0.574, 0.371, 0, 0}, {12.1, 0.689, 0.929, 0.134, 3.85}}}};
+
+// index of a call's weight kind in the tables
+int time_kind(const Problem& P) { return P.wk != WK_W4 ? 0 : P.hz ? 2 : 1; }
 
 double tile_time(const Problem& P, const SkArgs& a, int tile, int M, int S) {
-  const TileTime& m = kTileTime[P.wk == WK_W4][P.nsets - 1][tile];
+  const TileTime& m = kTileTime[time_kind(P)][P.nsets - 1][tile];
   int bm, bn;
   prefill_i8_geometry(tile, &bm, &bn);
   const long long wgs = (long long)((M + bm - 1) / bm) * col_tiles(P, a, bn) * S;
@@ -170,15 +187,16 @@ double tile_time(const Problem& P, const SkArgs& a, int tile, int M, int S) {
   const long long full = wgs / (256LL * m.cap), rest = wgs - full * 256LL * m.cap;
   double st = (double)full * m.s[m.cap - 1];
   if (rest > 0) st += m.s[(rest + 255) / 256 - 1];
-  double t = m.t0 + st * nst * (P.hz ? kZerosFactor : 1.0);
+  const double weights = (double)P.K * P.ncols * P.nsets * (P.wk == WK_W4 ? 0.5e-6 : 1e-6);
+  double t = m.t0 + st * nst + m.wmb * weights;
   if (S > 1) t += m.xs * S + m.xmb * 1e-6 * (double)wgs * bm * bn * 4 * P.nsets;
   return t;
 }
 
 double rows_time(const Problem& P, const SkArgs& a, int M, int S) {
-  const RowsTime& m = kRowsTime[P.wk == WK_W4][P.nsets - 1][S > 1];
+  const RowsTime& m = kRowsTime[time_kind(P)][P.nsets - 1][S > 1];
   const double w = (double)((M + 15) / 16) * col_tiles(P, a, S > 1 ? 128 : 64) * S / 256.0;
-  return m.t0 + (P.K / 64 / S / 2) * (m.c0 + m.c1 * std::max(1.0, w)) * (P.hz ? 1.15 : 1.0) + m.xs * S + m.xw * w;
+  return m.t0 + (P.K / 64 / S / 2) * (m.c0 + m.c1 * std::max(1.0, w)) + m.xs * S + m.xw * w;
 }
 
 // Rows per launch that `cap` bytes of partial tiles and the arrival counters hold, in

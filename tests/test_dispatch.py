@@ -37,3 +37,15 @@ def test_calls_without_a_split_need_no_workspace(tmp_path):
                                             ((D.gemm_i8, 2048, 512), (D.gemm_i8, 2048, 2048), (D.gate_up_w4, 512, 256),
                                              (D.gate_up_w4, 2048, 6144))]):
         assert st == 0 and events, msg
+
+
+@pytest.mark.parametrize("call,kernel", [
+    # gemm_i8 4096x12288 at 96 rows: 28.3 us on 128x128, 36 on the 64-column tiles
+    (D.gemm_i8(96, 4096, 12288), "prefill_i8_kernelILi0ELb0ELi0ELi4ELi2E"),
+    (D.gemm_i8(512, 12288, 4096), "prefill_i8_kernelILi0ELb0ELi0ELi4ELi2E"),
+    # W4 2048x6144 at 129 rows: 19.6 us on the 16-row tiles, 20.5 on 96x64, two rows of tiles
+    (D.gemm_w4(129, 2048, 6144), "skinny_kernel"),
+    (D.gate_up_i8(64, 2048, 2048), "prefill_i8_kernelILi0ELb0ELi2ELi2ELi1E"),
+])
+def test_engine_tiles(tmp_path, call, kernel):
+    assert kernel in _grid(D.run(tmp_path, [call])[0])[1]
