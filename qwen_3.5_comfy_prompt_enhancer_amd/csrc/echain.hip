@@ -1074,36 +1074,40 @@ std::vector<EPlanInfo> g_eplans;
 // The single-call form: up to 3 jobs (same K, activations, weight format) at level 0,
 // split-K scratch from the caller's workspace ([counters | partials]).  `clear` zeroes
 // the counters first (a scratch not known to be zero).
-// Workgroups of a single call's grid that are resident on the device at once.
-int g_cres[64][2];
+// The kernel of a call: of one job or more, of a weight format, with or without polling.
+template <int NJ>
+using ECall = void (*)(const ECallArgs<NJ>);
+template <int NJ>
+ECall<NJ> ecall_fn(bool w4, bool poll) {
+  if (w4) return poll ? ecall_kernel<true, true, NJ> : ecall_kernel<true, false, NJ>;
+  return poll ? ecall_kernel<false, true, NJ> : ecall_kernel<false, false, NJ>;
+}
+
+// Workgroups of a call's grid that are resident on the device at once, of the polling form
+// that would be launched: the forms are compiled apart, and a grid that one of them holds
+// another need not.
+int g_cres[64][2][2];
+template <int NJ>
 int ecall_resident(bool w4, int* n) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess || dev < 0 || dev >= 64) return set_error(QLIN_ERR_HIP, "echain_call: hipGetDevice failed");
   std::lock_guard<std::mutex> lk(g_emu);
-  if (g_cres[dev][w4] == 0) {
+  int& res = g_cres[dev][w4][NJ > 1];
+  if (res == 0) {
     int cus = 0, per = 0;
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-      e = w4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ecall_kernel<true, true, 3>, ET, 0)
-             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ecall_kernel<false, true, 3>, ET, 0);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ecall_fn<NJ>(w4, true), ET, 0);
     if (e != hipSuccess || cus <= 0 || per <= 0) return set_error(QLIN_ERR_HIP, "echain_call: occupancy query failed");
-    g_cres[dev][w4] = cus * per;
+    res = cus * per;
   }
-  *n = g_cres[dev][w4];
+  *n = res;
   return QLIN_OK;
 }
 
 template <int NJ>
 void ecall_launch(bool w4, bool poll, const ECallArgs<NJ>& a, hipStream_t stream) {
-  const dim3 grid((unsigned)a.nunits), block(ET);
-  if (w4) {
-    if (poll) hipLaunchKernelGGL((ecall_kernel<true, true, NJ>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((ecall_kernel<true, false, NJ>), grid, block, 0, stream, a);
-  } else {
-    if (poll) hipLaunchKernelGGL((ecall_kernel<false, true, NJ>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((ecall_kernel<false, false, NJ>), grid, block, 0, stream, a);
-  }
+  hipLaunchKernelGGL(ecall_fn<NJ>(w4, poll), dim3((unsigned)a.nunits), dim3(ET), 0, stream, a);
 }
 
 // The workspace (or a scratch laid out like it): `counter_bytes` of arrival counters,
@@ -1141,7 +1145,7 @@ int echain_call(const char* fn, EJob* jobs, int njobs, int M, void* ws, size_t w
   bool poll = false;
   if (parts > 0) {
     int resident = 0;
-    QL_TRY_E(ecall_resident(w4, &resident));
+    QL_TRY_E(njobs == 1 ? ecall_resident<1>(w4, &resident) : ecall_resident<3>(w4, &resident));
     const char* ep = getenv("QLIN_ECALL_POLL");
     poll = !(ep && strcmp(ep, "0") == 0) && ws && units <= resident && (size_t)parts * 4 <= poll_bytes &&
            wsb >= counter_bytes + poll_bytes;

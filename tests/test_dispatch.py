@@ -49,3 +49,14 @@ def test_calls_without_a_split_need_no_workspace(tmp_path):
 ])
 def test_engine_tiles(tmp_path, call, kernel):
     assert kernel in _grid(D.run(tmp_path, [call])[0])[1]
+
+
+@pytest.mark.parametrize("call", [D.gemm_i8(1, 2048, 2048), D.gemm_w4(4, 2048, 2048), D.gate_up_w4(1, 2048, 2048),
+                                  D.proj3_i8(1, 2048, 1024, 512, 512)])
+def test_residency_is_asked_of_the_kernel_that_polls(tmp_path, call):
+    """A call's split tiles poll their partners, which is safe if every workgroup of the
+    launched kernel is resident at once: the occupancy asked for is that kernel's."""
+    st, events, msg = D.run(tmp_path, [call])[0]
+    assert st == 0, msg
+    assert [e[0] for e in events] == ["occupancy", "launch"]
+    assert events[0][1] == events[1][1]
