@@ -785,6 +785,10 @@ __global__ __launch_bounds__(ET) __attribute__((amdgpu_waves_per_eu(3))) void ec
   const int u = blockIdx.x;
   int jn = 0;
   if constexpr (NJ > 1) jn = (a.njobs > 1 && u >= a.jobs[1].unit0) + (a.njobs > 2 && u >= a.jobs[2].unit0);
+  // (W4: with the job's place known the compiler loads every field at once, 25 scalar registers
+  // too many, and spills: 12288x4096 at 4 rows 16.6 us against 16.1, 6144x2048 at one 10.3 against
+  // 10.0.  W8 has room for them: 5 % faster so.)
+  else if constexpr (W4 && POLL) asm volatile("" : "+s"(jn));
   const EJob& J = a.jobs[jn];
   const EPos P = unit_pos(J, jn, u);
   const int M = a.M;

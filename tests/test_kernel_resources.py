@@ -67,3 +67,10 @@ def test_prefill_tiles_do_not_spill_in_their_loops():
     outside it."""
     for k in _find("prefill_i8_kernel"):
         assert k[".vgpr_spill_count"] <= 3, (k[".name"], k[".vgpr_spill_count"])
+
+
+def test_polling_w4_calls_use_no_scratch():
+    """ecall_kernel<W4, polling, jobs>, one job and three."""
+    for part in ("Lb1ELb1ELi1E", "Lb1ELb1ELi3E"):
+        for k in _find("ecall_kernelI" + part):
+            assert k[".private_segment_fixed_size"] == 0 and k[".sgpr_spill_count"] == 0, k[".name"]
