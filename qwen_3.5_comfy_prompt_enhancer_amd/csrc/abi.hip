@@ -930,8 +930,17 @@ struct KgTime {
 constexpr KgTime kKgTime[2][2] = {  // [W8, W4][32, 64 rows]
     {{3.8, {0.27, 0.46, 0.73}, 0.0206, 0.36, 0.41, 0.42, 3}, {4.5, {0.30, 0.62, 0}, 0.0243, 0.28, 0.43, 0.37, 2}},
     {{4.0, {0.37, 0.44, 0.65}, 0.0149, 0.11, 0.40, 0.41, 3}, {4.8, {0.46, 0.68, 0}, 0.0133, 0.13, 0.42, 0.41, 2}}};
-// (larger grids were measured behind the large tiles, which re-read less)
+// (larger grids were measured behind the large tiles, which re-read less; a W4 call that may
+// not use those takes them: 80 such calls of up to 4000 workgroups 1.49x the 16-row tiles on
+// average, none slower)
 constexpr long long kKgWorkgroups = 1024;
+// Above the rows of the fit the model is up to a third below what runs (more tiles of few
+// steps each).  Measured there at 518 calls of 513-4096 rows against the plans without this
+// kernel: W8 takes it where it is 17 % ahead instead of 10 (8 calls were up to 21 % slower for
+// it, now 2 of them up to 12; K = 1280, N = 1248 at 1323 rows 16.7 us, 15.0 on 128x128 tiles),
+// and a W4 round of two 64-row workgroups to a CU costs what it does with many tiles.
+constexpr int kKgRows = 512;
+constexpr double kKgManyRowsW4 = 0.82;
 
 // The best short-prompt plan of a call: its time in seconds (negative if there is none).
 double plan_kg(int wk, int M, int K, int N, size_t part_cap, long long most, PfPlan* plan) {
@@ -948,8 +957,10 @@ double plan_kg(int wk, int M, int K, int N, size_t part_cap, long long most, PfP
       if (S > 1 && (part > (double)part_cap || tiles > (long long)(kCounterBytes / sizeof(unsigned)))) break;
       const int steps = (K / 32 + 4 * S - 1) / (4 * S);
       const long long full = wgs / (256LL * m.cap), rest = wgs - full * 256LL * m.cap;
-      double st = (double)full * m.s[m.cap - 1];
-      if (rest > 0) st += m.s[(rest + 255) / 256 - 1];
+      double s[3] = {m.s[0], m.s[1], m.s[2]};
+      if (wk == WK_W4 && bm == 64 && M > kKgRows) s[1] = kKgManyRowsW4;
+      double st = (double)full * s[m.cap - 1];
+      if (rest > 0) st += s[(rest + 255) / 256 - 1];
       const double t = m.t0 + steps * st + m.mb * mb + (S > 1 ? m.x0 + m.xs * S + m.xmb * part * 1e-6 : 0.0);
       if (best < 0.0 || t * 1e-6 < best) best = t * 1e-6, *plan = PfPlan{true, 0, S, 0, bm};
     }
@@ -1062,7 +1073,7 @@ PfPlan plan_prefill(int wk, int M, int K, int N, size_t part_cap, bool force_til
   // that much): 2048x2048 at M = 128 13.6 -> 8.1 us (W8), 6144x2048 21.5 -> 13.3 (W4)
   PfPlan kg;
   const double t_kg = plan_kg(wk, M, K, N, part_cap, large ? kKgWorkgroups : 1LL << 20, &kg);
-  if (t_kg >= 0.0 && t_kg < 0.9 * best_t) return kg;
+  if (t_kg >= 0.0 && t_kg < (!w4 && M > kKgRows ? 0.83 : 0.9) * best_t) return kg;
   return best;
 }
 

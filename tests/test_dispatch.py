@@ -60,3 +60,16 @@ def test_residency_is_asked_of_the_kernel_that_polls(tmp_path, call):
     assert st == 0, msg
     assert [e[0] for e in events] == ["occupancy", "launch"]
     assert events[0][1] == events[1][1]
+
+
+@pytest.mark.parametrize("call,kernel", [
+    # above the rows that the short-prompt kernel's model is fitted on (512) it was chosen
+    # where it is slower: 16.7 us against 15.0, 16.5 / 15.2, 24.9 / 21.1
+    (D.linear_w8(1323, 1280, 1248), "prefill_kernel"), (D.linear_w8(1500, 1280, 1248), "prefill_kernel"),
+    (D.linear_w4(4000, 2048, 512), "prefill_kernel"),
+    # and where it stays the faster one: 8.6 us against 9.5, 16.6 / 18.8
+    (D.linear_w8(513, 512, 2048), "prefill_kg_kernel"), (D.linear_w8(1500, 4096, 320), "prefill_kg_kernel"),
+    (D.linear_w8(128, 2048, 2048), "prefill_kg_kernel"), (D.linear_w4(128, 6144, 2048), "prefill_kg_kernel"),
+])
+def test_short_prompt_kernel_choice(tmp_path, call, kernel):
+    assert kernel in _grid(D.run(tmp_path, [call])[0])[1]
