@@ -136,12 +136,14 @@ __global__ void requant_w4_kernel(const float* __restrict__ w, int K, int N, int
   sbf[(long long)gi * N + n] = f32_to_bf16(sc);
 }
 
-// W8 in one pass (N % 4 == 0): a workgroup of 1024 threads owns a strip of 4 L columns.
+// W8 in one launch (N % 4 == 0): a workgroup of 1024 threads owns a strip of 4 L columns.
 // Thread (q = tid / L) holds 4 columns of rows q, q + 1024 / L, ... in registers (NIT of
 // them; the rows past those are read again from the caches for the second half), the
-// columns' amax meets in LDS, and the codes are written from the registers.  Bound by HBM,
-// and by a workgroup's read and write phases not overlapping (its registers hold one
-// workgroup per CU).  K = 4096, N = 12288: 76 us, 4096 x 4096: 25 us, 2048 x 2048: 9.0 us,
+// columns' amax meets in LDS, and the codes are written from the registers: 512 rows of the
+// wide form <8, 16>, 1024 / 2048 / 4096 of <4, 4> / <8, 4> / <16, 4>, whose last 12 spill.
+// Bound by HBM and the second read of the other rows (7/8 of 4096 in the wide form, about
+// 1 MB a strip), and by a workgroup's read and write phases not overlapping (its registers
+// hold one workgroup per CU).  K = 4096, N = 12288: 76 us, 4096 x 4096: 25 us, 2048 x 2048: 9.0 us,
 // against 110 / 48.5 / 30 us in four launches (amax by atomics, codes with a division
 // each, scale).
 template <int NIT, int L>
@@ -217,6 +219,21 @@ __global__ void w8_amax_kernel(const float* __restrict__ w, int K, int N, int ro
   atomicMax(bits + n, bitcast<unsigned>(amax));
 }
 
+// the same, 4 columns per thread (N % 4 == 0)
+__global__ void w8_amax_x4_kernel(const float* __restrict__ w, int K, int N, int rows, unsigned* __restrict__ bits) {
+  const int n = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+  if (n >= N) return;
+  const int r0 = blockIdx.y * rows, r1 = min(K, r0 + rows);
+  f32x4 amax = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = r0; r < r1; ++r) {
+    const f32x4 v = *(const f32x4*)(w + (long long)r * N + n);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) amax[c] = fmaxf(amax[c], fabsf(v[c]));
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) atomicMax(bits + n + c, bitcast<unsigned>(amax[c]));
+}
+
 __global__ void fill_u32_kernel(unsigned* __restrict__ p, int n, unsigned v) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -231,6 +248,25 @@ __global__ void w8_quant_kernel(const float* __restrict__ w, int K, int N, const
     const int n = (int)(i % N);
     const float sc = fmaxf(bitcast<float>(bits[n]), 1e-8f) / 127.0f;
     q[i] = (int8_t)(int)fminf(fmaxf(rintf(w[i] / sc), -127.0f), 127.0f);
+  }
+}
+
+// the same, 4 consecutive elements per thread (N % 4 == 0, so they share a row)
+__global__ void w8_quant_x4_kernel(const float* __restrict__ w, int K, int N, const unsigned* __restrict__ bits,
+                                   int8_t* __restrict__ q) {
+  const long long total4 = (long long)K * N / 4;
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total4;
+       i += (long long)gridDim.x * blockDim.x) {
+    const int n = (int)((4 * i) % N);
+    const f32x4 v = *(const f32x4*)(w + 4 * i);
+    const u32x4 b = *(const u32x4*)(bits + n);
+    uint32_t word = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float sc = fmaxf(bitcast<float>(b[c]), 1e-8f) / 127.0f;
+      word |= ((uint32_t)(int)fminf(fmaxf(rintf(v[c] / sc), -127.0f), 127.0f) & 0xFFu) << (8 * c);
+    }
+    *(uint32_t*)(q + 4 * i) = word;
   }
 }
 
@@ -412,7 +448,14 @@ hipError_t launch_requant_w4(const float* w, int K, int N, int group, uint8_t* p
 }
 
 hipError_t launch_requant_w8(const float* w, int K, int N, int8_t* q, float* scale, hipStream_t st) {
-  if (N % 4 == 0 && aligned16(w) && aligned16(q) && aligned16(scale)) {
+  const bool x4 = N % 4 == 0 && aligned16(w) && aligned16(q) && aligned16(scale);
+  // Longer columns take four launches that spread the rows over the chip: a strip walks all
+  // of them on one CU, twice past its registers, from farther caches the longer it is, and a
+  // second round of strips starts late.  us, strips / four launches: K = 16384: N = 64 45 / 34,
+  // 1024 89 / 66, 4096 162 / 144; K = 12288: 1024 53 / 50, 4096 104 / 112, 6144 185 / 156;
+  // K = 8192: 64 24 / 24, 4096 66 / 83, 8192 155 / 135; K = 6144: 6144 82 / 90.
+  const int longest = N <= 256 ? 8192 : N <= 2048 ? 10240 : N < 6144 ? 12288 : 6144;
+  if (x4 && K <= longest) {
     // 64 columns per strip where that leaves at least 128 strips, or where a strip's rows fit
     // the registers twice over; 16 columns otherwise (K = 4096: N = 6144 38 us against 46
     // with 64 columns, N = 8192 65 against 53, N = 16384 150 against 110; K = 1024, N = 6144
@@ -430,9 +473,15 @@ hipError_t launch_requant_w8(const float* w, int K, int N, int8_t* q, float* sca
   const unsigned cb = (unsigned)((N + 255) / 256);
   constexpr int kRows = 64;  // rows per amax block: enough blocks to fill the chip
   hipLaunchKernelGGL(fill_u32_kernel, dim3(cb), dim3(256), 0, st, bits, N, 0u);
-  hipLaunchKernelGGL(w8_amax_kernel, dim3(cb, (unsigned)((K + kRows - 1) / kRows)), dim3(256), 0, st, w, K, N, kRows,
-                     bits);
-  hipLaunchKernelGGL(w8_quant_kernel, grid_for((long long)K * N), dim3(256), 0, st, w, K, N, bits, q);
+  const unsigned rb = (unsigned)((K + kRows - 1) / kRows);
+  if (x4) {
+    hipLaunchKernelGGL(w8_amax_x4_kernel, dim3((unsigned)((N / 4 + 255) / 256), rb), dim3(256), 0, st, w, K, N, kRows,
+                       bits);
+    hipLaunchKernelGGL(w8_quant_x4_kernel, grid_for((long long)K * N / 4), dim3(256), 0, st, w, K, N, bits, q);
+  } else {
+    hipLaunchKernelGGL(w8_amax_kernel, dim3(cb, rb), dim3(256), 0, st, w, K, N, kRows, bits);
+    hipLaunchKernelGGL(w8_quant_kernel, grid_for((long long)K * N), dim3(256), 0, st, w, K, N, bits, q);
+  }
   hipLaunchKernelGGL(w8_scale_kernel, dim3(cb), dim3(256), 0, st, N, bits);
   return hipGetLastError();
 }

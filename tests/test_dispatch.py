@@ -73,3 +73,12 @@ def test_residency_is_asked_of_the_kernel_that_polls(tmp_path, call):
 ])
 def test_short_prompt_kernel_choice(tmp_path, call, kernel):
     assert kernel in _grid(D.run(tmp_path, [call])[0])[1]
+
+
+@pytest.mark.parametrize("K,N,launches", [(8192, 64, 1), (12288, 64, 4), (10240, 1024, 1), (16384, 1024, 4),
+                                          (12288, 4096, 1), (16384, 4096, 4), (6144, 8192, 1), (8192, 8192, 4)])
+def test_requant_long_columns(tmp_path, K, N, launches):
+    """Strips of columns for short columns, four launches over the rows for long ones (K = 16384,
+    N = 1024 89 us in strips, 66 in four launches; K = 6144, N = 8192 95 / 106)."""
+    st, events, msg = D.run(tmp_path, [D.requant_w8(K, N)])[0]
+    assert st == 0 and len(events) == launches, msg

@@ -24,7 +24,7 @@ def _weights(K, N, seed):
 
 
 @pytest.mark.parametrize("K,N", [(64, 4), (200, 20), (1030, 36), (2100, 516), (4130, 64), (300, 4100), (600, 8260),
-                                 (65, 7)])
+                                 (65, 7), (8200, 20), (12300, 516)])
 def test_requant_w8(K, N):
     from qwen35_amd.kernels import layout
     w = _weights(K, N, K + N)
