@@ -1175,7 +1175,8 @@ int a16_linear(const char* fn, int wk, const void* x, int x_dtype, int M, int K,
             (p.splits > 1 && (tiles * p.splits * waves * 128 * 64 * sizeof(float) > part_cap ||
                               tiles > kCounterBytes / sizeof(unsigned))))
           return fail(QLIN_ERR_UNSUPPORTED, "%s: QLIN_PREFILL_SPLITS=%d unusable here", fn, p.splits);
-        if (p.sk != 0 && (p.sk < 0 || p.splits != 1 || !prefill_balanced_ok((long long)tiles, K / 64, p.sk) ||
+        // (the 128x384 tile has no balanced schedule)
+        if (p.sk != 0 && (p.sk < 0 || p.splits != 1 || p.shape == PF_128x384 || !prefill_balanced_ok((long long)tiles, K / 64, p.sk) ||
                           tiles * 2 * waves * 128 * 64 * sizeof(float) > part_cap ||
                           tiles > kCounterBytes / sizeof(unsigned)))
           return fail(QLIN_ERR_UNSUPPORTED, "%s: QLIN_PREFILL_SK=%d unusable here", fn, p.sk);

@@ -662,7 +662,9 @@ static hipError_t launch_prefill_t(const TlArgs& a, hipStream_t st) {
 
 
 // One plan shape of one weight kind / zeros / scale dtype; the balanced schedule is
-// its own instantiation, so the other plans compile as they would without it.
+// its own instantiation, so the other plans compile as they would without it.  The planner
+// takes it on 256x256 alone; on 128x128, with one and two K groups, it is there for
+// QLIN_PREFILL_SK and the tests of the schedule at sizes that 256x256 has too few tiles for.
 template <int WK, bool HZ, int SD>
 static hipError_t launch_prefill_kind(const TlArgs& a, int shape, hipStream_t st) {
   const bool bal = a.sk > 0;

@@ -82,3 +82,13 @@ def test_requant_long_columns(tmp_path, K, N, launches):
     N = 1024 89 us in strips, 66 in four launches; K = 6144, N = 8192 95 / 106)."""
     st, events, msg = D.run(tmp_path, [D.requant_w8(K, N)])[0]
     assert st == 0 and len(events) == launches, msg
+
+
+@pytest.mark.parametrize("shape,refused", [(1, False), (2, False), (3, True)])
+def test_balanced_schedule_of_the_wide_tile_is_refused(tmp_path, shape, refused):
+    """QLIN_PREFILL_SK with the 128x384 tile, which has no balanced schedule, is refused with
+    a message before anything is launched (300 rows, 32 K tiles, 37 per workgroup)."""
+    st, events, msg = D.run(tmp_path, [D.linear_w8(300, 2048, 1280)],
+                            {"QLIN_PREFILL": "tiled", "QLIN_PREFILL_SHAPE": str(shape), "QLIN_PREFILL_SK": "37"})[0]
+    assert (st, not events) == ((-2, True) if refused else (0, False)), msg
+    assert ("QLIN_PREFILL_SK" in msg) == refused
