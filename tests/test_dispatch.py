@@ -92,3 +92,13 @@ def test_balanced_schedule_of_the_wide_tile_is_refused(tmp_path, shape, refused)
                             {"QLIN_PREFILL": "tiled", "QLIN_PREFILL_SHAPE": str(shape), "QLIN_PREFILL_SK": "37"})[0]
     assert (st, not events) == ((-2, True) if refused else (0, False)), msg
     assert ("QLIN_PREFILL_SK" in msg) == refused
+
+
+def test_forced_tiles_are_different_kernels(tmp_path):
+    """QLIN_I8_TILE, which the tests of equal bits across tiles set, picks five kernels."""
+    calls = [D.gemm_i8(300, 1984, 1280), D.proj3_i8(300, 1984, 1024, 256, 256)]
+    seen = [set(), set()]
+    for tile in range(5):
+        for i, r in enumerate(D.run(tmp_path, calls, {"QLIN_ENGINE_PREFILL": "tiled", "QLIN_I8_TILE": str(tile)})):
+            seen[i].add(_grid(r)[1])
+    assert [len(s) for s in seen] == [5, 5]

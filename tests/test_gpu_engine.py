@@ -454,11 +454,11 @@ def test_prefill_tiled_tile_order_does_not_change_results(splits, tiled):
 
 
 @pytest.mark.parametrize("splits,K", [(1, 2048), (2, 2048), (4, 2048), (1, 1984)])
-def test_prefill_tiled_dma_tile_same_bits(splits, K, tiled):
-    """The 4-wave 128 x 64 DMA tile (QLIN_I8_DMA=1) and the 8-wave 128 x 128 tile (the
-    default) fold every output in the same order: gemm_i8 with the residual and proj3
-    (three column segments) give the same bits on both, also with an odd number of
-    64-wide blocks (the last stage holds one block)."""
+def test_prefill_tiled_tile_shapes_same_bits(splits, K, tiled):
+    """Every tile shape of the tiled int8 kernel (QLIN_I8_TILE: 128 x 128, then 64, 96, 128
+    and 160 rows x 64 columns) folds every output in the same order: gemm_i8 with the
+    residual and proj3 (three column segments) give the same bits on all, also with an odd
+    number of 64-wide blocks (the last stage holds one block)."""
     gemm, _ = _g()
     tiled.setenv("QLIN_ENGINE_SPLITS", str(splits))
     M = 300
@@ -467,8 +467,8 @@ def test_prefill_tiled_dma_tile_same_bits(splits, K, tiled):
     ws = [H.engine_w8(K, n, seed=522 + i) for i, n in enumerate((1024, 256, 256))]
     hid = torch.randn((M, 1280), generator=H.gen(525)).to(torch.bfloat16).cuda()
     outs = []
-    for dma in ("1", "0"):
-        tiled.setenv("QLIN_I8_DMA", dma)
+    for tile in range(5):
+        tiled.setenv("QLIN_I8_TILE", str(tile))
         y = torch.empty((M, 1280), dtype=torch.bfloat16, device="cuda")
         gemm.gemm_i8(a.cuda(), as_.cuda(), b.cuda(), bs.cuda(), y, residual=hid)
         p3 = torch.empty((M, 1536), dtype=torch.bfloat16, device="cuda")
