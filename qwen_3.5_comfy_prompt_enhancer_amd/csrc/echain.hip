@@ -779,16 +779,19 @@ __device__ __forceinline__ void unit_loop(const EJob& J, const EPos& P, int M, E
 // Single call: unit u = blockIdx.x of up to 3 jobs (proj3 segments; one job otherwise).
 // POLL: every unit of the grid is resident at once, and split tiles use the polling
 // exchange on slots that start zero and are left zero.
-template <bool W4, bool POLL, int NJ>
+// LATE: a single job's descriptor through an index that the compiler cannot fold.  With its
+// place known every field is loaded at once, which for W4 takes 25 scalar registers too many
+// and spills them.  Without a producer that costs (12288x4096 at 4 rows 16.6 us against 16.1,
+// 6144x2048 at one 10.3 against 10.0); behind a producer the early loads are still worth it (a
+// W4 2048-hidden layer's four fused calls at 4 rows, six layers: 271 us against 276).  W8 has
+// room for the fields: 5 % faster so.
+template <bool W4, bool POLL, int NJ, bool LATE = false>
 __global__ __launch_bounds__(ET) __attribute__((amdgpu_waves_per_eu(3))) void ecall_kernel(const ECallArgs<NJ> a) {
   __shared__ ESh sh;
   const int u = blockIdx.x;
   int jn = 0;
   if constexpr (NJ > 1) jn = (a.njobs > 1 && u >= a.jobs[1].unit0) + (a.njobs > 2 && u >= a.jobs[2].unit0);
-  // (W4: with the job's place known the compiler loads every field at once, 25 scalar registers
-  // too many, and spills: 12288x4096 at 4 rows 16.6 us against 16.1, 6144x2048 at one 10.3 against
-  // 10.0.  W8 has room for them: 5 % faster so.)
-  else if constexpr (W4 && POLL) asm volatile("" : "+s"(jn));
+  else if constexpr (LATE) asm volatile("" : "+s"(jn));
   const EJob& J = a.jobs[jn];
   const EPos P = unit_pos(J, jn, u);
   const int M = a.M;
@@ -1078,11 +1081,14 @@ std::vector<EPlanInfo> g_eplans;
 // The single-call form: up to 3 jobs (same K, activations, weight format) at level 0,
 // split-K scratch from the caller's workspace ([counters | partials]).  `clear` zeroes
 // the counters first (a scratch not known to be zero).
-// The kernel of a call: of one job or more, of a weight format, with or without polling.
+// The kernel of a call: of one job or more, of a weight format, with or without polling,
+// with the descriptor's loads late (W4 single jobs that poll).
 template <int NJ>
 using ECall = void (*)(const ECallArgs<NJ>);
 template <int NJ>
-ECall<NJ> ecall_fn(bool w4, bool poll) {
+ECall<NJ> ecall_fn(bool w4, bool poll, bool late) {
+  if constexpr (NJ == 1)
+    if (w4 && poll && late) return ecall_kernel<true, true, 1, true>;
   if (w4) return poll ? ecall_kernel<true, true, NJ> : ecall_kernel<true, false, NJ>;
   return poll ? ecall_kernel<false, true, NJ> : ecall_kernel<false, false, NJ>;
 }
@@ -1090,18 +1096,18 @@ ECall<NJ> ecall_fn(bool w4, bool poll) {
 // Workgroups of a call's grid that are resident on the device at once, of the polling form
 // that would be launched: the forms are compiled apart, and a grid that one of them holds
 // another need not.
-int g_cres[64][2][2];
+int g_cres[64][2][2][2];
 template <int NJ>
-int ecall_resident(bool w4, int* n) {
+int ecall_resident(bool w4, bool late, int* n) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess || dev < 0 || dev >= 64) return set_error(QLIN_ERR_HIP, "echain_call: hipGetDevice failed");
   std::lock_guard<std::mutex> lk(g_emu);
-  int& res = g_cres[dev][w4][NJ > 1];
+  int& res = g_cres[dev][w4][NJ > 1][late];
   if (res == 0) {
     int cus = 0, per = 0;
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ecall_fn<NJ>(w4, true), ET, 0);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ecall_fn<NJ>(w4, true, late), ET, 0);
     if (e != hipSuccess || cus <= 0 || per <= 0) return set_error(QLIN_ERR_HIP, "echain_call: occupancy query failed");
     res = cus * per;
   }
@@ -1110,8 +1116,8 @@ int ecall_resident(bool w4, int* n) {
 }
 
 template <int NJ>
-void ecall_launch(bool w4, bool poll, const ECallArgs<NJ>& a, hipStream_t stream) {
-  hipLaunchKernelGGL(ecall_fn<NJ>(w4, poll), dim3((unsigned)a.nunits), dim3(ET), 0, stream, a);
+void ecall_launch(bool w4, bool poll, bool late, const ECallArgs<NJ>& a, hipStream_t stream) {
+  hipLaunchKernelGGL(ecall_fn<NJ>(w4, poll, late), dim3((unsigned)a.nunits), dim3(ET), 0, stream, a);
 }
 
 // The workspace (or a scratch laid out like it): `counter_bytes` of arrival counters,
@@ -1147,9 +1153,10 @@ int echain_call(const char* fn, EJob* jobs, int njobs, int M, void* ws, size_t w
   for (int i = njobs; i < 3 && njobs > 1; ++i) memset(&a.jobs[i], 0, sizeof(EJob));
   if (units > 0x7FFFFFFFLL) return set_error(QLIN_ERR_UNSUPPORTED, "echain_call: grid too large");
   bool poll = false;
+  const bool late = w4 && njobs == 1 && a.jobs[0].pro.kind == PRO_NONE;
   if (parts > 0) {
     int resident = 0;
-    QL_TRY_E(njobs == 1 ? ecall_resident<1>(w4, &resident) : ecall_resident<3>(w4, &resident));
+    QL_TRY_E(njobs == 1 ? ecall_resident<1>(w4, late, &resident) : ecall_resident<3>(w4, late, &resident));
     const char* ep = getenv("QLIN_ECALL_POLL");
     poll = !(ep && strcmp(ep, "0") == 0) && ws && units <= resident && (size_t)parts * 4 <= poll_bytes &&
            wsb >= counter_bytes + poll_bytes;
@@ -1184,9 +1191,9 @@ int echain_call(const char* fn, EJob* jobs, int njobs, int M, void* ws, size_t w
     b.pad = 0;
     b.part = a.part;
     b.cnt = a.cnt;
-    ecall_launch(w4, poll, b, stream);
+    ecall_launch(w4, poll, late, b, stream);
   } else {
-    ecall_launch(w4, poll, a, stream);
+    ecall_launch(w4, poll, late, a, stream);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {

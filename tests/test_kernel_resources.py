@@ -70,7 +70,8 @@ def test_prefill_tiles_do_not_spill_in_their_loops():
 
 
 def test_polling_w4_calls_use_no_scratch():
-    """ecall_kernel<W4, polling, jobs>, one job and three."""
-    for part in ("Lb1ELb1ELi1E", "Lb1ELb1ELi3E"):
+    """ecall_kernel<W4, polling, jobs, late>: the form of calls without a producer, and of
+    three jobs (a single call behind a producer loads its descriptor early, and spills)."""
+    for part in ("Lb1ELb1ELi1ELb1E", "Lb1ELb1ELi3ELb0E"):
         for k in _find("ecall_kernelI" + part):
             assert k[".private_segment_fixed_size"] == 0 and k[".sgpr_spill_count"] == 0, k[".name"]
