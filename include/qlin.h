@@ -28,7 +28,7 @@
  * kernels need N % 16 == 0 (per projection), 16-byte aligned weights, scales, zeros,
  * outputs and residuals, 16-bit row strides that are multiples of 8, and 8-byte
  * aligned a_q; a call outside those rules runs on a generic kernel (same arithmetic
- * per block, one K split).  The A16 entry points (qlin_linear_*)
+ * per block, K split over the eight waves of a workgroup).  The A16 entry points (qlin_linear_*)
  * and the chains keep the fast rules and refuse other layouts.
  */
 #ifndef QLIN_H

@@ -295,10 +295,9 @@ __device__ __forceinline__ int round_i8(float v) {
 // round_i8(y / s) for inv = 1 / s and |y| <= 127 s up to rounding: y * inv is within 4e-5
 // of the quotient there, and so is the sum with 0.5, so wherever the product lies further
 // than 1e-4 from a tie the nearest integer is the code; the others (2 in 10000) divide.
-// Seven instructions against fifteen or more.  With the butterflies below: six W8
-// 2048-hidden layers at one row as engine chains 265.4 -> 263.0 us, a W4 layer's fused calls
-// at 4 rows 274.4 -> 270.9 (six layers), its linears and producers at 512 rows 131.6 -> 130.5
-// (W8), at 137 rows 216.7 -> 214.8 (W4, 4096 hidden).
+// Seven instructions against fifteen or more.  With the butterflies below about 1 % of a layer,
+// at the edge of what two runs differ by: six W8 2048-hidden layers at one row as engine chains
+// 265.4 -> 263.0 us, a W8 layer's linears and producers at 512 rows 131.6 -> 130.5.
 __device__ __forceinline__ int quant_i8(float y, float s, float inv) {
   const float v = y * inv;
   const float r = rintf(v);
