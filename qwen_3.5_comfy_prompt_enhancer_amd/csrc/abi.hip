@@ -1033,6 +1033,9 @@ PfPlan plan_tiled(int wk, int M, int K, int N, size_t part_cap, double* t) {
 // weights, where the 16-row tiles and the short-prompt kernel multiply fp32 dots by them, so
 // calls on the 16-row tiles' side of this line (their time against tiles of 128x128 and
 // 256x256, microseconds) keep the fp32 form.
+// The line is fixed: it decides the arithmetic of a call, not which tile is the fastest, so its
+// constants stay as they are when plan_tiled's are fitted again.  It takes the workspace into
+// account as the splits of the large tiles do: a smaller one can move a call to the fp32 side.
 bool w4_large_tiles(int M, int K, int N, size_t part_cap) {
   const double row_wgs = (double)((M + 15) / 16) * ((N + 127) / 128);
   const double t_rows = 5.8 + std::max(1.0, row_wgs / 256) * 2.7e-3 * K;
